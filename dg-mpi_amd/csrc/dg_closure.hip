@@ -852,7 +852,9 @@ void closure_steps(dg_solver* s, dg_mlp* m, double dt, double bound, int nsteps,
         a.dt = dt;
         a.alpha = alpha;
         a.mode = mode;
-        hcheck(dg::launch_stage_corrected(s->P, (int)s->cfg.flux, a, C, s->dtab, s->geo, s->stream),
+        const int flux = (int)s->cfg.flux;
+        hcheck(s->faces ? dg::launch_stage_two_pass(s->P, flux, a, s->faces, C, s->dtab, s->geo, s->stream)
+                        : dg::launch_stage_corrected(s->P, flux, a, C, s->dtab, s->geo, s->stream),
                "corrected stage kernel");
     };
     for (int k = 0; k < nsteps; ++k) {

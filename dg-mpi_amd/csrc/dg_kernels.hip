@@ -3062,6 +3062,7 @@ __global__ __launch_bounds__(256) void mass_kernel(double* imm, double* jmin, co
 }
 
 #include "dg_kernels_2d.inc"
+#include "dg_stage_split.inc"
 
 // ---------------------------------------------------------------------------
 // Dispatch
@@ -3120,6 +3121,48 @@ hipError_t stage_p(int flux, const StageArgs& a, const KTables* t, const KGeom& 
         }
     }
     return hipGetLastError();
+}
+
+// The two passes of an RK stage (dg_stage_split.inc); Corr: the closure's
+// correction (p = 1, FP64) or null
+template <int P, class R, bool CORR>
+hipError_t two_pass_elements(const StageArgs& a, const R* faces, const KTables* t, const KGeom& g, const BoxDiv& dv,
+                             const float* corr, hipStream_t st) {
+    using Dm = ElemDims<P, R>;
+    const dim3 grid((((g.E + Dm::EPB - 1) / Dm::EPB) + 7u) & ~7u), block(Dm::TS);
+    switch (a.mode) {
+    case MODE_RK_FIRST: hipLaunchKernelGGL((element_kernel<P, R, MODE_RK_FIRST, CORR>), grid, block, 0, st, a, faces, t, g, dv, corr); break;
+    case MODE_RK_MID: hipLaunchKernelGGL((element_kernel<P, R, MODE_RK_MID, CORR>), grid, block, 0, st, a, faces, t, g, dv, corr); break;
+    case MODE_RK_LAST: hipLaunchKernelGGL((element_kernel<P, R, MODE_RK_LAST, CORR>), grid, block, 0, st, a, faces, t, g, dv, corr); break;
+    case MODE_FE:
+        if constexpr (!CORR) {
+            hipLaunchKernelGGL((element_kernel<P, R, MODE_FE, false>), grid, block, 0, st, a, faces, t, g, dv, corr);
+            break;
+        }
+        return hipErrorInvalidValue;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+template <int P, class R>
+hipError_t two_pass_p(int flux, const StageArgs& a, void* scratch, const float* corr, const KTables* t, const KGeom& g,
+                      hipStream_t st) {
+    using Dm = FaceDims<P, R>;
+    const dim3 grid((((g.E + Dm::EPB - 1) / Dm::EPB) + 7u) & ~7u), block(WAVE);
+    const BoxDiv dv = make_box_div(g);
+    R* faces = static_cast<R*>(scratch);
+    switch (flux) {
+    case 0: hipLaunchKernelGGL((face_flux_kernel<P, 0, R>), grid, block, 0, st, a.Ust, faces, t, g, dv); break;
+    case 1: hipLaunchKernelGGL((face_flux_kernel<P, 1, R>), grid, block, 0, st, a.Ust, faces, t, g, dv); break;
+    default: hipLaunchKernelGGL((face_flux_kernel<P, 2, R>), grid, block, 0, st, a.Ust, faces, t, g, dv); break;
+    }
+    if (const hipError_t e = hipGetLastError()) return e;
+    if constexpr (P == 1 && sizeof(R) == 8) {
+        if (corr) return two_pass_elements<P, R, true>(a, faces, t, g, dv, corr, st);
+    }
+    if (corr) return hipErrorInvalidValue;
+    return two_pass_elements<P, R, false>(a, faces, t, g, dv, nullptr, st);
 }
 
 template <int P, int TS, int PROJ>
@@ -3232,6 +3275,28 @@ hipError_t launch_stage(int P, int flux, const StageArgs& a, const KTables* t, c
         DG_DISPATCH_P(P, return stage2d_p<PP>(flux, a, t, g, st));
     }
     DG_DISPATCH_P(P, return stage_p<PP>(flux, a, t, g, st));
+    return hipSuccess;
+}
+
+// Elements from which the two passes beat the fused stage, whose single
+// launch is the shorter one while launches and latency count (us of a middle
+// stage, two passes / fused, at the sizes on either side: p = 1 4096
+// 12.1 / 11.8, 8000 15.5 / 20.7; p = 2 1728 16.4 / 12.3, 4096 19.4 / 23.3;
+// p = 3 1728 24.7 / 20.3, 4096 34.6 / 38.4)
+unsigned two_pass_min_elements(int P) {
+    static const unsigned lim[PMAX] = {4608, 2560, 2816, 2816, 2816};
+    return P >= 1 && P <= PMAX ? lim[P - 1] : ~0u;
+}
+
+size_t two_pass_scratch_bytes(int P, const KGeom& g, unsigned elements) {
+    if (g.dim != 3 || g.mapped || g.fp32 || P < 1 || P > PMAX || elements < two_pass_min_elements(P)) return 0;
+    return (size_t)g.E * FACE_OUT(P) * sizeof(double);
+}
+
+hipError_t launch_stage_two_pass(int P, int flux, const StageArgs& a, void* scratch, const float* corr,
+                                 const KTables* t, const KGeom& g, hipStream_t st) {
+    if (!scratch || g.dim != 3 || g.mapped || g.fp32 || a.mode == MODE_RESIDUAL) return hipErrorInvalidValue;
+    DG_DISPATCH_P(P, return (two_pass_p<PP, double>(flux, a, scratch, corr, t, g, st)));
     return hipSuccess;
 }
 

@@ -121,6 +121,26 @@ struct StageArgs {
     int mode;
 };
 
+// Multipliers of box_xyz (element number -> box coordinates, dg_stage_split.inc)
+struct BoxDiv {
+    unsigned mx, sx, my, sy;
+};
+inline void box_div(unsigned d, unsigned& m, unsigned& s) {
+    m = s = 0;
+    if (d <= 1) return;
+    while ((2ull << s) < d) ++s;
+    m = (unsigned)(((1ull << (32 + s)) + d - 1) / d);
+}
+inline BoxDiv make_box_div(const KGeom& g) {
+    BoxDiv v;
+    box_div((unsigned)g.ne[0], v.mx, v.sx);
+    box_div((unsigned)g.ne[1], v.my, v.sy);
+    return v;
+}
+// values per element of the two-pass stage's scratch array (the lifted
+// fluxes of the three - faces)
+constexpr int FACE_OUT(int P) { return 3 * NVAR * (P + 1) * (P + 1); }
+
 // One case of a batched stage launch (device memory): its RK registers as
 // byte offsets from the base pointer the launch receives (pointers derived
 // from a kernel argument are known to the compiler to be global memory,
@@ -140,6 +160,15 @@ struct BatchCase {
 // `t` points to the case's KTables in device memory.
 hipError_t launch_stage(int P, int flux, const StageArgs& a, const KTables* t, const KGeom& g,
                         hipStream_t st);
+// The same RK stage (not the residual) in two passes, for the affine box in
+// FP64: every face's lifted flux once into `scratch`, then
+// the rest.  two_pass_scratch_bytes: the bytes of scratch for the case, 0
+// where launch_stage is the better one for a launch over `elements` elements
+// (the case's own, or all of a batch group) or the only one.  corr: the
+// correction of launch_stage_corrected, or null.
+size_t two_pass_scratch_bytes(int P, const KGeom& g, unsigned elements);
+hipError_t launch_stage_two_pass(int P, int flux, const StageArgs& a, void* scratch, const float* corr,
+                                 const KTables* t, const KGeom& g, hipStream_t st);
 // RK stage of an affine FP64 p = 1 box with dU = dt (M^-1 R + C): C the
 // learned closure's FP32 correction, laid out like the state.
 hipError_t launch_stage_corrected(int P, int flux, const StageArgs& a, const float* C, const KTables* t,

@@ -109,6 +109,13 @@ double max_wavespeed(dg_solver* s, const double* U) {
     return m;
 }
 
+// an RK or forward-Euler stage in the form the handle was set up for
+hipError_t launch_rk_stage(dg_solver* s, const dg::StageArgs& a) {
+    const int flux = (int)s->cfg.flux;
+    if (s->faces) return dg::launch_stage_two_pass(s->P, flux, a, s->faces, nullptr, s->dtab, s->geo, s->stream);
+    return dg::launch_stage(s->P, flux, a, s->dtab, s->geo, s->stream);
+}
+
 // one time step of the configured stepper on U0 (stream-ordered)
 void step_once(dg_solver* s, double dt) {
     using namespace dg;
@@ -116,13 +123,12 @@ void step_once(dg_solver* s, double dt) {
     a.dt = dt;
     a.cmp = s->cmp;
     hipStream_t st = s->stream;
-    const int flux = (int)s->cfg.flux;
     if (s->cfg.stepper == Stepper::FE) {
         // the stage reads neighbours of U0 while other elements update, so
         // the new state goes to Ua and is copied back (the state pointer
         // handed out by dg_state_device_ptr stays valid)
         a.Ust = s->U0; a.U0 = s->U0; a.Uout = s->Ua; a.mode = MODE_FE;
-        hip_check(launch_stage(s->P, flux, a, s->dtab, s->geo, st), "stage kernel");
+        hip_check(launch_rk_stage(s, a), "stage kernel");
         hip_check(hipMemcpyAsync(s->U0, s->Ua, s->ncoef * sizeof(double), hipMemcpyDeviceToDevice, st),
                   "hipMemcpyAsync");
         s->time += dt;
@@ -131,15 +137,15 @@ void step_once(dg_solver* s, double dt) {
     // RK4 (src/numerics/timestepping/stepper.cpp:71-142), fused stages
     a.U0 = s->U0; a.acc = s->acc;
     a.Ust = s->U0; a.Uout = s->Ua; a.alpha = 0.5; a.mode = MODE_RK_FIRST;
-    hip_check(launch_stage(s->P, flux, a, s->dtab, s->geo, st), "stage kernel");
+    hip_check(launch_rk_stage(s, a), "stage kernel");
     s->time += dt / 2.0;
     a.Ust = s->Ua; a.Uout = s->Ub; a.alpha = 0.5; a.mode = MODE_RK_MID;
-    hip_check(launch_stage(s->P, flux, a, s->dtab, s->geo, st), "stage kernel");
+    hip_check(launch_rk_stage(s, a), "stage kernel");
     a.Ust = s->Ub; a.Uout = s->Ua; a.alpha = 1.0; a.mode = MODE_RK_MID;
-    hip_check(launch_stage(s->P, flux, a, s->dtab, s->geo, st), "stage kernel");
+    hip_check(launch_rk_stage(s, a), "stage kernel");
     s->time += dt / 2.0;
     a.Ust = s->Ua; a.Uout = s->U0; a.mode = MODE_RK_LAST;
-    hip_check(launch_stage(s->P, flux, a, s->dtab, s->geo, st), "stage kernel");
+    hip_check(launch_rk_stage(s, a), "stage kernel");
 }
 
 // a new state starts without carried rounding error
@@ -194,6 +200,8 @@ void free_all(dg_solver* s) {
         if (p) (void)hipFree(p);
     if (s->cmp) (void)hipFree(s->cmp);
     s->cmp = nullptr;
+    if (s->faces) (void)hipFree(s->faces);
+    s->faces = nullptr;
     if (s->frec) (void)hipFree(s->frec);
     s->frec = nullptr;
     s->nev = nullptr;
@@ -296,6 +304,13 @@ int create(const char* toml_text, const MeshInput* mesh, dg_solver** out) {
         if (cfg.compensated) {
             hip_check(hipMalloc(&s->cmp, s->ncoef * sizeof(float)), "hipMalloc(cmp)");
             hip_check(dg::launch_zero(s->cmp, s->ncoef * sizeof(float), s->stream), "zero kernel (cmp)");
+        }
+        if (const size_t fb = dg::two_pass_scratch_bytes(s->P, s->geo, s->geo.E)) {
+            // a case that fits the device without the scratch runs without it
+            if (hipMalloc(&s->faces, fb) != hipSuccess) {
+                (void)hipGetLastError();
+                s->faces = nullptr;
+            }
         }
         if (s->geo.mapped) {
             // upload the general-path tables, then form the per-element

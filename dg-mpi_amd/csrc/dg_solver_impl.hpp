@@ -28,6 +28,7 @@ struct dg_solver {
     double* Ub = nullptr;
     double* acc = nullptr;             // RK accumulator
     float* cmp = nullptr;              // Stepper.compensated: rounding error of U0 (FP32)
+    void* faces = nullptr;             // scratch of the two-pass stage (null: the fused stage)
     double* work = nullptr;            // per-element reduction output
     double* X = nullptr;               // mapped box: element node coordinates [E][8][3]
     double* imm = nullptr;             // mapped box: inverse mass matrices [E][nb][nb]

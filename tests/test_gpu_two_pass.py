@@ -1,0 +1,111 @@
+"""Boxes large enough for the two-pass RK stage (faces once, then the
+elements): one RK4 and one forward-Euler step against the steps composed from
+the residual and inverse-mass calls, which run the fused kernel on the same
+state.  Element counts just above the size where the two passes take over
+(and one below), with every remainder of the workgroups' element counts among
+them, single-element directions (an element that is its own neighbour), all
+orders, bases and fluxes."""
+import numpy as np
+import pytest
+
+import dg_amd
+from dg_amd import hip
+
+pytestmark = pytest.mark.gpu
+
+# order, elements: p = 1 takes over at 4608 elements, p = 2 at 2560, the rest
+# at 2816; the workgroups of the two passes hold 7 and 6, 5 and 4, 4 and 5,
+# 3 and 3, 3 and 2 elements
+CASES = [
+    (1, (17, 17, 16), "LegendreHex", "Roe"), (1, (19, 16, 25), "LagrangeHex", "HLLC"),
+    (2, (14, 15, 13), "LagrangeHex", "LaxFriedrichs"), (2, (17, 19, 17), "LegendreHex", "Roe"),
+    (2, (1, 2561, 1), "LegendreHex", "HLLC"),
+    (3, (17, 13, 13), "LegendreHex", "Roe"), (3, (2819, 1, 1), "LagrangeHex", "HLLC"),
+    (3, (14, 14, 14), "LegendreHex", "LaxFriedrichs"), (3, (18, 18, 18), "LagrangeHex", "Roe"),
+    (4, (15, 14, 14), "LegendreHex", "HLLC"), (4, (23, 22, 23), "LagrangeHex", "Roe"),
+    (5, (15, 15, 13), "LegendreHex", "Roe"), (5, (19, 19, 19), "LagrangeHex", "LaxFriedrichs"),
+]
+
+
+def solver(order, ne, basis, flux, stepper="RK4", precision=None):
+    dt = 0.02 / max(ne) / (2 * order + 1)
+    # unequal element widths; the vortex stays resolved by the small boxes
+    s = dg_amd.Solver(dg_amd.case_toml(order=order, basis=basis, flux=flux, nelem=ne, lower=(-5., -4., -3.),
+                                       upper=(5., 4., 3.), stepper=stepper, timestep=dt, precision=precision,
+                                       ic="ExtrudedIsentropicVortex", ic_data=(1.0, 0.7, -0.4, 1.0, 3.0, 0.3, -0.2)))
+    s.init_state_from_fcn()
+    return s, dt
+
+
+def composed(s, U0, dt, stepper):
+    """a step from get_residual and mult_inv_mass_matrix on buffers of the host's own"""
+    n = U0.size
+    u, r = hip.Buffer(n), hip.Buffer(n)
+
+    def tendency(U):
+        u.upload(U)
+        s.get_residual(u.addr, r.addr)
+        s.mult_inv_mass_matrix(dt, r.addr, r.addr)
+        hip.synchronize()
+        return r.download(U.shape)
+
+    k1 = tendency(U0)
+    if stepper == "FE":
+        out = U0 + k1
+    else:
+        k2 = tendency(U0 + 0.5 * k1)
+        k3 = tendency(U0 + 0.5 * k2)
+        k4 = tendency(U0 + k3)
+        out = U0 + (k1 + 2.0 * k2 + 2.0 * k3 + k4) / 6.0
+    u.free()
+    r.free()
+    return out
+
+
+@pytest.mark.parametrize("order,ne,basis,flux", CASES)
+@pytest.mark.parametrize("precision", [None, "FP32"])
+def test_step_matches_the_composed_step(order, ne, basis, flux, precision):
+    print(f"two-pass p={order} {ne} {basis} {flux} {precision}", flush=True)
+    for stepper in ("RK4", "FE"):
+        s, dt = solver(order, ne, basis, flux, stepper, precision)
+        with s:
+            U0 = s.get_state()
+            s.take_time_step()
+            U1 = s.get_state()
+            ref = composed(s, U0, dt, stepper)
+        d = np.max(np.abs(U1 - ref))
+        # the increment carries the form's rounding: 2^-53 (2^-24) per
+        # operation over some hundreds of operations and the growth of M^-1,
+        # (2 p + 1)^3 between the modes; the state adds its own last place
+        inc = np.max(np.abs(ref - U0))
+        eps = 2.0 ** -53 if precision is None else 2.0 ** -24
+        tol = 64 * eps * (2 * order + 1) ** 3 * inc + 4 * 2.0 ** -52 * np.max(np.abs(ref))
+        assert np.all(np.isfinite(U1)) and inc > 0.0
+        assert d <= tol, (stepper, d, tol, inc)
+
+
+@pytest.mark.parametrize("precision", [None, "FP32"])
+def test_integrals_are_conserved(precision):
+    s, _ = solver(3, (18, 18, 18), "LegendreHex", "Roe", "RK4", precision)
+    with s:
+        I0 = s.integrals()
+        s.take_time_step(0.0, 20)
+        I1 = s.integrals()
+    bar = 1e-13 if precision is None else 1e-6
+    assert np.max(np.abs(I1[:5] - I0[:5])) <= bar * np.max(np.abs(I0[:5]))
+
+
+def test_closure_step_with_a_zero_network_is_the_plain_step():
+    from dg_amd import closure
+    m = closure.MLP(0)
+    p = m.params()
+    p[:] = 0.0
+    m.set_params(p)
+    a, _ = solver(1, (17, 17, 16), "LegendreHex", "Roe")
+    b, _ = solver(1, (17, 17, 16), "LegendreHex", "Roe")
+    with a, b:
+        a.take_time_step(0.0, 2)
+        closure.step(b, m, 1e30, 2)
+        Ua, Ub = a.get_state(), b.get_state()
+    m.close()
+    assert np.max(np.abs(Ua - Ub)) <= 4 * 2.0 ** -52 * np.max(np.abs(Ua))
