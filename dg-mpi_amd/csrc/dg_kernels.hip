@@ -3280,22 +3280,36 @@ hipError_t launch_stage(int P, int flux, const StageArgs& a, const KTables* t, c
 
 // Elements from which the two passes beat the fused stage, whose single
 // launch is the shorter one while launches and latency count (us of a middle
-// stage, two passes / fused, at the sizes on either side: p = 1 4096
+// stage, two passes / fused, at the sizes on either side: FP64 p = 1 4096
 // 12.1 / 11.8, 8000 15.5 / 20.7; p = 2 1728 16.4 / 12.3, 4096 19.4 / 23.3;
-// p = 3 1728 24.7 / 20.3, 4096 34.6 / 38.4)
-unsigned two_pass_min_elements(int P) {
-    static const unsigned lim[PMAX] = {4608, 2560, 2816, 2816, 2816};
-    return P >= 1 && P <= PMAX ? lim[P - 1] : ~0u;
+// p = 3 1728 24.7 / 20.3, 4096 34.6 / 38.4; FP32 p = 1 4096 12.4 / 10.2, 8000
+// 15.0 / 15.7; p = 2 4096 18.3 / 17.6, 8000 24.2 / 29.6; p = 4 19600 185 /
+// 183, 32768 281 / 384; p = 5 4096 81 / 79, 8000 145 / 151).  The FP32 form at
+// p = 3 stays fused: there stage_kernel solves in the box's frame, and the
+// two passes' FP32 rounding would differ from it (at the other orders the
+// two agree to the bit).
+unsigned two_pass_min_elements(int P, int fp32) {
+    static const unsigned lim[2][PMAX] = {{4608, 2560, 2816, 2816, 2816}, {7168, 5120, ~0u, 24576, 6656}};
+    return P >= 1 && P <= PMAX ? lim[fp32 ? 1 : 0][P - 1] : ~0u;
 }
 
 size_t two_pass_scratch_bytes(int P, const KGeom& g, unsigned elements) {
-    if (g.dim != 3 || g.mapped || g.fp32 || P < 1 || P > PMAX || elements < two_pass_min_elements(P)) return 0;
-    return (size_t)g.E * FACE_OUT(P) * sizeof(double);
+    if (g.dim != 3 || g.mapped || g.proj || P < 1 || P > PMAX || elements < two_pass_min_elements(P, g.fp32)) return 0;
+    return (size_t)g.E * FACE_OUT(P) * (g.fp32 ? sizeof(float) : sizeof(double));
 }
 
 hipError_t launch_stage_two_pass(int P, int flux, const StageArgs& a, void* scratch, const float* corr,
                                  const KTables* t, const KGeom& g, hipStream_t st) {
-    if (!scratch || g.dim != 3 || g.mapped || g.fp32 || a.mode == MODE_RESIDUAL) return hipErrorInvalidValue;
+    if (!scratch || g.dim != 3 || g.mapped || g.proj || a.mode == MODE_RESIDUAL) return hipErrorInvalidValue;
+    if (g.fp32) {
+        switch (P) {
+        case 1: return two_pass_p<1, float>(flux, a, scratch, corr, t, g, st);
+        case 2: return two_pass_p<2, float>(flux, a, scratch, corr, t, g, st);
+        case 4: return two_pass_p<4, float>(flux, a, scratch, corr, t, g, st);
+        case 5: return two_pass_p<5, float>(flux, a, scratch, corr, t, g, st);
+        default: return hipErrorInvalidValue;
+        }
+    }
     DG_DISPATCH_P(P, return (two_pass_p<PP, double>(flux, a, scratch, corr, t, g, st)));
     return hipSuccess;
 }
