@@ -3061,8 +3061,8 @@ __global__ __launch_bounds__(256) void mass_kernel(double* imm, double* jmin, co
     team_for<NB * NB, TS>(lane, [&](int t) { imm[(size_t)e * NB * NB + t] = A[t]; });
 }
 
-#include "dg_kernels_2d.inc"
 #include "dg_stage_split.inc"
+#include "dg_kernels_2d.inc"
 
 // ---------------------------------------------------------------------------
 // Dispatch
