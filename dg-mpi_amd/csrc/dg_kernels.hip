@@ -394,7 +394,8 @@ __device__ __forceinline__ void riemann_roe(R gam, const R* UL, const R* UR, R n
 // uref[s] of the reference state by selects on values (a dynamic index,
 // or a select of the members' addresses, would copy the kernel-argument
 // struct to scratch memory)
-__device__ __forceinline__ double uref_of(const KGeom& G, int s) {
+template <class GEO>
+__device__ __forceinline__ double uref_of(GEO& G, int s) {
     const double u0 = G.uref[0], u1 = G.uref[1], u2 = G.uref[2], u3 = G.uref[3], u4 = G.uref[4];
     return s == 0 ? u0 : (s == 1 ? u1 : (s == 2 ? u2 : (s == 3 ? u3 : u4)));
 }
@@ -422,8 +423,8 @@ struct SplitRef {
     }
 };
 
-template <class R>
-__device__ __forceinline__ SplitRef<R> split_ref(const KGeom& G) {
+template <class R, class GEO>
+__device__ __forceinline__ SplitRef<R> split_ref(GEO& G) {
     SplitRef<R> r;
     r.rho = R(G.uref[0]);
 #pragma unroll
@@ -3165,6 +3166,26 @@ hipError_t two_pass_p(int flux, const StageArgs& a, void* scratch, const float* 
     return two_pass_elements<P, R, false>(a, faces, t, g, dv, nullptr, st);
 }
 
+template <int P, class R>
+hipError_t two_pass_batch_p(int flux, BatchCase* cases, const unsigned* face_case, unsigned face_blocks,
+                            const unsigned* elem_case, unsigned elem_blocks, int stage, const KTables* t,
+                            hipStream_t st) {
+    char* base = reinterpret_cast<char*>(cases);
+    const dim3 fgrid((face_blocks + 7u) & ~7u), egrid((elem_blocks + 7u) & ~7u), eblock(ElemDims<P, R>::TS);
+    switch (flux) {
+    case 0: hipLaunchKernelGGL((face_flux_batch_kernel<P, 0, R>), fgrid, dim3(WAVE), 0, st, cases, face_case, face_blocks, stage, t, base); break;
+    case 1: hipLaunchKernelGGL((face_flux_batch_kernel<P, 1, R>), fgrid, dim3(WAVE), 0, st, cases, face_case, face_blocks, stage, t, base); break;
+    default: hipLaunchKernelGGL((face_flux_batch_kernel<P, 2, R>), fgrid, dim3(WAVE), 0, st, cases, face_case, face_blocks, stage, t, base); break;
+    }
+    if (const hipError_t e = hipGetLastError()) return e;
+    switch (stage) {
+    case 0: hipLaunchKernelGGL((element_batch_kernel<P, R, MODE_RK_FIRST>), egrid, eblock, 0, st, cases, elem_case, elem_blocks, stage, t, base); break;
+    case 3: hipLaunchKernelGGL((element_batch_kernel<P, R, MODE_RK_LAST>), egrid, eblock, 0, st, cases, elem_case, elem_blocks, stage, t, base); break;
+    default: hipLaunchKernelGGL((element_batch_kernel<P, R, MODE_RK_MID>), egrid, eblock, 0, st, cases, elem_case, elem_blocks, stage, t, base); break;
+    }
+    return hipGetLastError();
+}
+
 template <int P, int TS, int PROJ>
 hipError_t stage_batch_proj(int flux, const BatchCase* cases, const unsigned* blk_case, unsigned nblocks, int stage,
                             const KTables* t, hipStream_t st) {
@@ -3296,6 +3317,38 @@ unsigned two_pass_min_elements(int P, int fp32) {
 size_t two_pass_scratch_bytes(int P, const KGeom& g, unsigned elements) {
     if (g.dim != 3 || g.mapped || g.proj || P < 1 || P > PMAX || elements < two_pass_min_elements(P, g.fp32)) return 0;
     return (size_t)g.E * FACE_OUT(P) * (g.fp32 ? sizeof(float) : sizeof(double));
+}
+
+unsigned two_pass_blocks(int P, int fp32, int pass, unsigned E) {
+    unsigned epb = 1;
+    switch (P) {
+#define DG_EPB(PP)                                                                                   \
+    case PP:                                                                                         \
+        epb = fp32 ? (pass ? ElemDims<PP, float>::EPB : FaceDims<PP, float>::EPB)                    \
+                   : (pass ? ElemDims<PP, double>::EPB : FaceDims<PP, double>::EPB);                 \
+        break;
+        DG_EPB(1) DG_EPB(2) DG_EPB(3) DG_EPB(4) DG_EPB(5)
+#undef DG_EPB
+    }
+    return (E + epb - 1) / epb;
+}
+
+hipError_t launch_stage_two_pass_batch(int P, int flux, int fp32, BatchCase* cases, const unsigned* face_case,
+                                       unsigned face_blocks, const unsigned* elem_case, unsigned elem_blocks, int stage,
+                                       const KTables* t, hipStream_t st) {
+#define DG_TWO(PP, R) two_pass_batch_p<PP, R>(flux, cases, face_case, face_blocks, elem_case, elem_blocks, stage, t, st)
+    if (fp32) {
+        switch (P) {
+        case 1: return DG_TWO(1, float);
+        case 2: return DG_TWO(2, float);
+        case 4: return DG_TWO(4, float);
+        case 5: return DG_TWO(5, float);
+        default: return hipErrorInvalidValue;
+        }
+    }
+    DG_DISPATCH_P(P, return DG_TWO(PP, double));
+#undef DG_TWO
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_stage_two_pass(int P, int flux, const StageArgs& a, void* scratch, const float* corr,

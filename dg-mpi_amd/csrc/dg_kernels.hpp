@@ -153,6 +153,11 @@ struct BatchCase {
     double dt;
     KGeom g;
     unsigned first_block;
+    // two-pass stage: the case's share of the group's scratch array, and its
+    // first workgroup in the sequences of the face and of the element pass
+    long long off_faces;
+    BoxDiv dv;
+    unsigned first_face, first_elem;
 };
 
 // Launchers; P in 1..PMAX, flux 0 LLF / 1 HLLC / 2 Roe.  Return the launch
@@ -179,6 +184,13 @@ hipError_t launch_stage_corrected(int P, int flux, const StageArgs& a, const flo
 // 0 or 1 picks one of two team sizes per order (batch_team).
 hipError_t launch_stage_batch(int P, int flux, int fp32, int proj, int variant, const BatchCase* cases,
                               const unsigned* blk_case, unsigned nblocks, int stage, const KTables* t, hipStream_t st);
+// The same stage in two passes (launch_stage_two_pass): workgroups of the
+// group and the case of each, for either pass; base: the cases array.
+// two_pass_blocks: workgroups of one pass (0 faces, 1 elements) over E elements.
+unsigned two_pass_blocks(int P, int fp32, int pass, unsigned E);
+hipError_t launch_stage_two_pass_batch(int P, int flux, int fp32, BatchCase* cases, const unsigned* face_case,
+                                       unsigned face_blocks, const unsigned* elem_case, unsigned elem_blocks, int stage,
+                                       const KTables* t, hipStream_t st);
 // threads per element of the batched launch's variant (0 or 1) at order P
 int batch_team(int P, int variant);
 // zero `bytes` (a multiple of 4) of device memory with a kernel on st

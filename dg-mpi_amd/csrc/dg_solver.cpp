@@ -679,6 +679,10 @@ struct dg_batch {
         std::vector<int> members;             // indices into cases
         dg::BatchCase* dcases = nullptr;      // device descriptors
         unsigned* blk_case = nullptr;         // device: case (within the group) of each block
+        // two-pass stage (faces != null; then blk_case holds the cases of the
+        // face pass's workgroups and, behind them, of the element pass's)
+        void* faces = nullptr;                // device: lifted fluxes of the group's faces
+        unsigned pass_blocks[2] = {0, 0};     // workgroups of the face and of the element pass
         int variant = 0;                      // team-size variant of the launch (dg::batch_team)
         int cap = BRICK_CAPS[0];              // log2 edge cap of the element bricks of its cases
         double ms[2] = {0.0, 0.0};            // one RK4 step with each team variant at the chosen cap
@@ -702,6 +706,20 @@ namespace {
 
 thread_local std::string g_batch_error;
 
+// a case's bytes of its group's two-pass scratch array (0: fused stage)
+size_t group_face_bytes(const dg_batch::Group& g, const dg_solver* s) {
+    return (dg::two_pass_scratch_bytes(g.P, s->geo, g.nblocks) + 255) & ~(size_t)255;
+}
+
+// one RK4 stage of a group
+hipError_t launch_group_stage(const dg_batch* b, const dg_batch::Group& g, int variant, int stage, hipStream_t st) {
+    const dg::KTables* t = b->cases[g.members[0]]->dtab;
+    if (g.faces)
+        return dg::launch_stage_two_pass_batch(g.P, g.flux, g.fp32, g.dcases, g.blk_case, g.pass_blocks[0],
+                                               g.blk_case + g.pass_blocks[0], g.pass_blocks[1], stage, t, st);
+    return dg::launch_stage_batch(g.P, g.flux, g.fp32, g.proj, variant, g.dcases, g.blk_case, g.nblocks, stage, t, st);
+}
+
 // descriptors of a group's cases: the case's registers (as byte offsets
 // from the descriptor array, the base the launch receives), dt, geometry
 void upload_group(dg_batch* b, dg_batch::Group& g) {
@@ -709,7 +727,8 @@ void upload_group(dg_batch* b, dg_batch::Group& g) {
     std::vector<BatchCase> h(g.members.size());
     const char* base = reinterpret_cast<const char*>(g.dcases);
     auto off = [&](const void* p) { return (long long)(reinterpret_cast<const char*>(p) - base); };
-    unsigned first = 0;
+    unsigned first = 0, first_pass[2] = {0, 0};
+    size_t face_bytes = 0;
     for (size_t k = 0; k < g.members.size(); ++k) {
         const dg_solver* s = b->cases[g.members[k]];
         BatchCase& c = h[k];
@@ -726,6 +745,14 @@ void upload_group(dg_batch* b, dg_batch::Group& g) {
         for (int d = 0; d < 3; ++d) c.g.tile[d] = std::min(s->geo.tile[d], g.cap);
         c.first_block = first;
         first += s->geo.E;
+        if (g.faces) {
+            c.off_faces = off(g.faces) + (long long)face_bytes;
+            face_bytes += group_face_bytes(g, s);
+            c.dv = make_box_div(s->geo);
+            c.first_face = first_pass[0];
+            c.first_elem = first_pass[1];
+            for (int p = 0; p < 2; ++p) first_pass[p] += two_pass_blocks(g.P, g.fp32, p, s->geo.E);
+        }
     }
     // ordered on the batch stream (the group branches of a step fork from it)
     hip_check(hipMemcpyAsync(g.dcases, h.data(), h.size() * sizeof(BatchCase), hipMemcpyHostToDevice, b->stream),
@@ -748,8 +775,7 @@ hipError_t launch_step(dg_batch* b) {
         hipStream_t st = branch ? g.stream : b->stream;
         if (branch) e = hipStreamWaitEvent(st, b->fork, 0);
         for (int k = 0; k < 4 && e == hipSuccess; ++k)
-            e = dg::launch_stage_batch(g.P, g.flux, g.fp32, g.proj, g.variant, g.dcases, g.blk_case, g.nblocks, k,
-                                       b->cases[g.members[0]]->dtab, st);
+            e = launch_group_stage(b, g, g.variant, k, st);
         if (e == hipSuccess && branch) e = hipEventRecord(g.done, st);
     }
     for (size_t gi = 1; gi < b->groups.size() && e == hipSuccess && !serial; ++gi)
@@ -777,7 +803,8 @@ void capture_step(dg_batch* b) {
 // fastest candidate.  Each output value is computed by one thread with the
 // same operations whatever the team size or the traversal order (each
 // variant being compiled on its own, multiply-add fusion may differ:
-// round-off), so these are ordinary steps of the cases.
+// round-off), so these are ordinary steps of the cases.  A group that runs
+// in two passes has one form: its fastest time stands for every candidate.
 constexpr int TUNE_STEPS = 2 + NCAND;
 
 void tune(dg_batch* b) {
@@ -798,9 +825,7 @@ void tune(dg_batch* b) {
             for (size_t gi = 0; gi < ng; ++gi) {
                 auto& g = b->groups[gi];
                 hip_check(hipEventRecord(ev[gi * 8 + st * 2], b->stream), "hipEventRecord");
-                hip_check(dg::launch_stage_batch(g.P, g.flux, g.fp32, g.proj, v, g.dcases, g.blk_case, g.nblocks, st,
-                                                 b->cases[g.members[0]]->dtab, b->stream),
-                          "batched stage launch");
+                hip_check(launch_group_stage(b, g, v, st, b->stream), "batched stage launch");
                 hip_check(hipEventRecord(ev[gi * 8 + st * 2 + 1], b->stream), "hipEventRecord");
             }
         hip_check(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
@@ -819,6 +844,7 @@ void tune(dg_batch* b) {
     for (auto& e : ev) (void)hipEventDestroy(e);
     for (auto& g : b->groups) {
         int best = 0;
+        if (g.faces) std::fill_n(g.ms_cand, NCAND, *std::min_element(g.ms_cand, g.ms_cand + NCAND));
         for (int c = 1; c < NCAND; ++c)
             if (g.ms_cand[c] < g.ms_cand[best]) best = c;
         g.variant = best & 1;
@@ -838,6 +864,7 @@ void free_batch(dg_batch* b) {
     for (auto& g : b->groups) {
         if (g.dcases) (void)hipFree(g.dcases);
         if (g.blk_case) (void)hipFree(g.blk_case);
+        if (g.faces) (void)hipFree(g.faces);
         if (g.stream) (void)hipStreamDestroy(g.stream);
         if (g.done) (void)hipEventDestroy(g.done);
     }
@@ -905,11 +932,22 @@ int dg_batch_create(int num_cases, dg_solver* const* cases, dg_batch** out) {
         }
         for (auto& g : b->groups) {
             hip_check(hipMalloc(&g.dcases, g.members.size() * sizeof(dg::BatchCase)), "hipMalloc(batch cases)");
-            hip_check(hipMalloc(&g.blk_case, (size_t)g.nblocks * sizeof(unsigned)), "hipMalloc(batch blocks)");
-            std::vector<unsigned> bc(g.nblocks);
-            size_t k = 0;
-            for (size_t m = 0; m < g.members.size(); ++m)
-                for (unsigned e = 0; e < b->cases[g.members[m]]->geo.E; ++e) bc[k++] = (unsigned)m;
+            size_t face_bytes = 0;
+            for (int m : g.members) face_bytes += group_face_bytes(g, b->cases[m]);
+            if (face_bytes && hipMalloc(&g.faces, face_bytes) != hipSuccess) {
+                (void)hipGetLastError();      // no room for the scratch: the fused stage needs none
+                g.faces = nullptr;
+            }
+            // the case of each workgroup, of one launch or of both passes
+            std::vector<unsigned> bc;
+            for (int p = 0; p < (g.faces ? 2 : 1); ++p) {
+                for (size_t m = 0; m < g.members.size(); ++m) {
+                    const unsigned E = b->cases[g.members[m]]->geo.E;
+                    bc.insert(bc.end(), g.faces ? dg::two_pass_blocks(g.P, g.fp32, p, E) : E, (unsigned)m);
+                }
+                if (g.faces) g.pass_blocks[p] = (unsigned)bc.size() - (p ? g.pass_blocks[0] : 0u);
+            }
+            hip_check(hipMalloc(&g.blk_case, bc.size() * sizeof(unsigned)), "hipMalloc(batch blocks)");
             hip_check(hipMemcpy(g.blk_case, bc.data(), bc.size() * sizeof(unsigned), hipMemcpyHostToDevice),
                       "hipMemcpy(batch blocks)");
             upload_group(b, g);

@@ -198,8 +198,10 @@ int dg_set_stream(dg_solver* s, void* stream);
  * (Stepper.timestep or the CFL-derived one) and time; after
  * dg_batch_step(b, n) every case holds what dg_step(case, 0, n) would have
  * produced (the same stage arithmetic; the compiler may fuse multiply-adds
- * differently in the batched kernel, which moves round-off only).  Cases: distinct handles on one device, 3D affine
- * boxes (no mesh, no warp), RK4.  The batch borrows the handles: destroy it
+ * differently in the batched kernel, and a group large enough takes its
+ * stages in two passes though a case of it alone would not: both move
+ * round-off only).  Cases: distinct handles on one device, 3D affine boxes
+ * (no mesh, no warp), RK4.  The batch borrows the handles: destroy it
  * before them.  dg_batch_step waits for each case's stream before it starts
  * and returns when the steps are done. */
 typedef struct dg_batch dg_batch;
@@ -215,7 +217,8 @@ const char* dg_batch_last_error(const dg_batch* b);
  * first dg_batch_step call with nsteps >= 6 runs its first six steps as
  * tuning steps (one with each team size, not counted: code loading; then
  * one with each candidate), keeps each group's fastest candidate and
- * captures the step again.  This reports, per group, the order, the team
+ * captures the step again.  A group that runs its stages in two passes has
+ * one form: its fastest step stands for every candidate.  This reports, per group, the order, the team
  * size in use and the two team sizes' timings at the chosen cap (ms per
  * RK4 step of the group run alone; 0 before tuning).  Arrays of
  * *num_groups entries; NULL arrays: only the count. */

@@ -111,3 +111,43 @@ def test_closure_step_with_a_zero_network_is_the_plain_step():
         Ua, Ub = a.get_state(), b.get_state()
     m.close()
     assert np.max(np.abs(Ua - Ub)) <= 4 * 2.0 ** -52 * np.max(np.abs(Ua))
+
+
+# cases of one batch: every order's group (and one in the FP32 form) is large
+# enough together, though no case is by itself; uneven sizes, so that the
+# workgroups' sequences end in every remainder, and single-element cases
+BATCH = [
+    (1, (13, 11, 17), "LegendreHex", "Roe", None), (1, (17, 17, 8), "LegendreHex", "Roe", None),
+    (2, (9, 9, 9), "LagrangeHex", "HLLC", None), (2, (13, 7, 5), "LagrangeHex", "HLLC", None),
+    (2, (1, 1, 1), "LagrangeHex", "HLLC", None), (2, (11, 12, 11), "LagrangeHex", "HLLC", None),
+    (3, (14, 14, 14), "LegendreHex", "LaxFriedrichs", None), (3, (3, 5, 7), "LegendreHex", "LaxFriedrichs", None),
+    (4, (13, 13, 13), "LegendreHex", "Roe", None), (4, (9, 9, 9), "LegendreHex", "Roe", None),
+    (5, (12, 12, 12), "LagrangeHex", "Roe", None), (5, (11, 11, 10), "LagrangeHex", "Roe", None),
+    (2, (15, 15, 15), "LegendreHex", "Roe", "FP32"), (2, (12, 13, 12), "LegendreHex", "Roe", "FP32"),
+]
+
+
+def test_batch_matches_each_case_alone():
+    made = [(solver(o, ne, b, f, "RK4", pr), solver(o, ne, b, f, "RK4", pr)) for o, ne, b, f, pr in BATCH]
+    batch_s, solo_s = [m[0][0] for m in made], [m[1][0] for m in made]
+    with dg_amd.Batch(batch_s) as batch:
+        for n in (1, 2, 7):          # replays of the captured step, then the tuned one
+            print(f"two-pass batch, {n} steps", flush=True)
+            before = [s.get_state() for s in solo_s]
+            for sb, U in zip(batch_s, before):
+                sb.set_state(U)
+            batch.step(n)
+            for (order, ne, _, _, prec), sb, so, U0 in zip(BATCH, batch_s, solo_s, before):
+                so.take_time_step(0.0, n)
+                ref, U1 = so.get_state(), sb.get_state()
+                # as above, over n steps
+                inc = np.max(np.abs(ref - U0))
+                eps = 2.0 ** -53 if prec is None else 2.0 ** -24
+                tol = n * (64 * eps * (2 * order + 1) ** 3 * inc + 4 * 2.0 ** -52 * np.max(np.abs(ref)))
+                d = np.max(np.abs(U1 - ref))
+                assert np.all(np.isfinite(U1)) and inc > 0.0
+                assert d <= tol, (order, ne, prec, n, d, tol)
+        for (cap, ncases, elements, ms) in batch.tiles():
+            assert min(ms) > 0.0 and cap in (2, 3)
+    for s in batch_s + solo_s:
+        s.close()
