@@ -793,7 +793,7 @@ void tendency(dg_solver* s, const double* U, double* D) {
     a.Ust = U;
     a.R = s->Ua;
     a.mode = dg::MODE_RESIDUAL;
-    hcheck(dg::launch_stage(s->P, (int)s->cfg.flux, a, s->dtab, s->geo, s->stream), "stage kernel");
+    hcheck(launch_solver_stage(s, a, nullptr, s->stream), "stage kernel");
     hcheck(dg::launch_inv_mass(s->P, 1.0, s->Ua, D, s->dtab, s->geo, s->stream), "inverse mass kernel");
 }
 
@@ -852,10 +852,7 @@ void closure_steps(dg_solver* s, dg_mlp* m, double dt, double bound, int nsteps,
         a.dt = dt;
         a.alpha = alpha;
         a.mode = mode;
-        const int flux = (int)s->cfg.flux;
-        hcheck(s->faces ? dg::launch_stage_two_pass(s->P, flux, a, s->faces, C, s->dtab, s->geo, s->stream)
-                        : dg::launch_stage_corrected(s->P, flux, a, C, s->dtab, s->geo, s->stream),
-               "corrected stage kernel");
+        hcheck(launch_solver_stage(s, a, C, s->stream), "corrected stage kernel");
     };
     for (int k = 0; k < nsteps; ++k) {
         // the stage kernel reads the neighbours of Ust: stages ping-pong

@@ -3141,6 +3141,12 @@ hipError_t two_pass_elements(const StageArgs& a, const R* faces, const KTables* 
             break;
         }
         return hipErrorInvalidValue;
+    case MODE_RESIDUAL:
+        if constexpr (!CORR) {
+            hipLaunchKernelGGL((element_kernel<P, R, MODE_RESIDUAL, false>), grid, block, 0, st, a, faces, t, g, dv, corr);
+            break;
+        }
+        return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -3305,10 +3311,11 @@ hipError_t launch_stage(int P, int flux, const StageArgs& a, const KTables* t, c
 // 12.1 / 11.8, 8000 15.5 / 20.7; p = 2 1728 16.4 / 12.3, 4096 19.4 / 23.3;
 // p = 3 1728 24.7 / 20.3, 4096 34.6 / 38.4; FP32 p = 1 4096 12.4 / 10.2, 8000
 // 15.0 / 15.7; p = 2 4096 18.3 / 17.6, 8000 24.2 / 29.6; p = 4 19600 185 /
-// 183, 32768 281 / 384; p = 5 4096 81 / 79, 8000 145 / 151).  The FP32 form at
-// p = 3 stays fused: there stage_kernel solves in the box's frame, and the
-// two passes' FP32 rounding would differ from it (at the other orders the
-// two agree to the bit).
+// 183, 32768 281 / 384; p = 5 4096 81 / 79, 8000 145 / 151; the residual in FP64
+// p = 1 4624 11.8 / 14.0, p = 2 2730 16.4 / 17.9, p = 5 2940 68.7 / 82.0).
+// The FP32 form at p = 3 stays fused: there stage_kernel solves in the box's
+// frame, and the two passes' FP32 rounding would differ from it (at the other
+// orders the two agree to the bit).
 unsigned two_pass_min_elements(int P, int fp32) {
     static const unsigned lim[2][PMAX] = {{4608, 2560, 2816, 2816, 2816}, {7168, 5120, ~0u, 24576, 6656}};
     return P >= 1 && P <= PMAX ? lim[fp32 ? 1 : 0][P - 1] : ~0u;
@@ -3353,7 +3360,7 @@ hipError_t launch_stage_two_pass_batch(int P, int flux, int fp32, BatchCase* cas
 
 hipError_t launch_stage_two_pass(int P, int flux, const StageArgs& a, void* scratch, const float* corr,
                                  const KTables* t, const KGeom& g, hipStream_t st) {
-    if (!scratch || g.dim != 3 || g.mapped || g.proj || a.mode == MODE_RESIDUAL) return hipErrorInvalidValue;
+    if (!scratch || g.dim != 3 || g.mapped || g.proj) return hipErrorInvalidValue;
     if (g.fp32) {
         switch (P) {
         case 1: return two_pass_p<1, float>(flux, a, scratch, corr, t, g, st);

@@ -165,7 +165,7 @@ struct BatchCase {
 // `t` points to the case's KTables in device memory.
 hipError_t launch_stage(int P, int flux, const StageArgs& a, const KTables* t, const KGeom& g,
                         hipStream_t st);
-// The same RK stage (not the residual) in two passes, for the affine box in
+// The same stage or residual in two passes, for the affine box in
 // FP64 and the FP32 form: every face's lifted flux once into `scratch`, then
 // the rest.  two_pass_scratch_bytes: the bytes of scratch for the case, 0
 // where launch_stage is the better one for a launch over `elements` elements

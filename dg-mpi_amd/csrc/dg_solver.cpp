@@ -109,13 +109,6 @@ double max_wavespeed(dg_solver* s, const double* U) {
     return m;
 }
 
-// an RK or forward-Euler stage in the form the handle was set up for
-hipError_t launch_rk_stage(dg_solver* s, const dg::StageArgs& a) {
-    const int flux = (int)s->cfg.flux;
-    if (s->faces) return dg::launch_stage_two_pass(s->P, flux, a, s->faces, nullptr, s->dtab, s->geo, s->stream);
-    return dg::launch_stage(s->P, flux, a, s->dtab, s->geo, s->stream);
-}
-
 // one time step of the configured stepper on U0 (stream-ordered)
 void step_once(dg_solver* s, double dt) {
     using namespace dg;
@@ -128,7 +121,7 @@ void step_once(dg_solver* s, double dt) {
         // the new state goes to Ua and is copied back (the state pointer
         // handed out by dg_state_device_ptr stays valid)
         a.Ust = s->U0; a.U0 = s->U0; a.Uout = s->Ua; a.mode = MODE_FE;
-        hip_check(launch_rk_stage(s, a), "stage kernel");
+        hip_check(launch_solver_stage(s, a, nullptr, s->stream), "stage kernel");
         hip_check(hipMemcpyAsync(s->U0, s->Ua, s->ncoef * sizeof(double), hipMemcpyDeviceToDevice, st),
                   "hipMemcpyAsync");
         s->time += dt;
@@ -137,15 +130,15 @@ void step_once(dg_solver* s, double dt) {
     // RK4 (src/numerics/timestepping/stepper.cpp:71-142), fused stages
     a.U0 = s->U0; a.acc = s->acc;
     a.Ust = s->U0; a.Uout = s->Ua; a.alpha = 0.5; a.mode = MODE_RK_FIRST;
-    hip_check(launch_rk_stage(s, a), "stage kernel");
+    hip_check(launch_solver_stage(s, a, nullptr, s->stream), "stage kernel");
     s->time += dt / 2.0;
     a.Ust = s->Ua; a.Uout = s->Ub; a.alpha = 0.5; a.mode = MODE_RK_MID;
-    hip_check(launch_rk_stage(s, a), "stage kernel");
+    hip_check(launch_solver_stage(s, a, nullptr, s->stream), "stage kernel");
     a.Ust = s->Ub; a.Uout = s->Ua; a.alpha = 1.0; a.mode = MODE_RK_MID;
-    hip_check(launch_rk_stage(s, a), "stage kernel");
+    hip_check(launch_solver_stage(s, a, nullptr, s->stream), "stage kernel");
     s->time += dt / 2.0;
     a.Ust = s->Ua; a.Uout = s->U0; a.mode = MODE_RK_LAST;
-    hip_check(launch_rk_stage(s, a), "stage kernel");
+    hip_check(launch_solver_stage(s, a, nullptr, s->stream), "stage kernel");
 }
 
 // a new state starts without carried rounding error
@@ -547,8 +540,7 @@ int dg_residual(dg_solver* s, const double* U_dev, double* R_dev, void* stream) 
         a.Ust = U_dev;
         a.R = R_dev;
         a.mode = dg::MODE_RESIDUAL;
-        hip_check(dg::launch_stage(s->P, (int)s->cfg.flux, a, s->dtab, s->geo, pick_stream(s, stream)),
-                  "stage kernel");
+        hip_check(launch_solver_stage(s, a, nullptr, pick_stream(s, stream)), "stage kernel");
     });
 }
 
@@ -653,6 +645,7 @@ int dg_set_stream(dg_solver* s, void* stream) {
     return guarded(s, [&] {
         need(s, "solver");
         set_device(s);
+        std::lock_guard<std::mutex> lk(s->faces_mu);
         hip_check(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
         s->stream = stream ? (hipStream_t)stream : s->own_stream;
     });

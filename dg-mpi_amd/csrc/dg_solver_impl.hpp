@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -29,6 +30,7 @@ struct dg_solver {
     double* acc = nullptr;             // RK accumulator
     float* cmp = nullptr;              // Stepper.compensated: rounding error of U0 (FP32)
     void* faces = nullptr;             // scratch of the two-pass stage (null: the fused stage)
+    std::mutex faces_mu;               // its two launches go to the stream as one
     double* work = nullptr;            // per-element reduction output
     double* X = nullptr;               // mapped box: element node coordinates [E][8][3]
     double* imm = nullptr;             // mapped box: inverse mass matrices [E][nb][nb]
@@ -44,3 +46,22 @@ struct dg_solver {
     std::vector<long> mesh_e2n;        // given mesh: element nodes [E][8] (2D: [E][4])
     std::string err;
 };
+
+// A stage or the residual of the handle's case; corr: the closure's
+// correction or null.  The two passes share the handle's scratch array: its
+// users are ordered by the handle's stream, each pair of launches enqueued
+// under the lock.  A residual on a stream of the caller's, or captured into
+// a graph that may be replayed on any stream, takes the fused kernel, which
+// needs no scratch.
+inline hipError_t launch_solver_stage(dg_solver* s, const dg::StageArgs& a, const float* corr, hipStream_t st) {
+    const int flux = (int)s->cfg.flux;
+    if (s->faces) {
+        std::lock_guard<std::mutex> lk(s->faces_mu);
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (a.mode != dg::MODE_RESIDUAL ||
+            (st == s->stream && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone))
+            return dg::launch_stage_two_pass(s->P, flux, a, s->faces, corr, s->dtab, s->geo, st);
+    }
+    if (corr) return dg::launch_stage_corrected(s->P, flux, a, corr, s->dtab, s->geo, st);
+    return dg::launch_stage(s->P, flux, a, s->dtab, s->geo, st);
+}

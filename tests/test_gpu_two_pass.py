@@ -42,12 +42,12 @@ def solver(order, ne, basis, flux, stepper="RK4", precision=None):
 def composed(s, U0, dt, stepper):
     """a step from get_residual and mult_inv_mass_matrix on buffers of the host's own"""
     n = U0.size
-    u, r = hip.Buffer(n), hip.Buffer(n)
+    u, r, st = hip.Buffer(n), hip.Buffer(n), hip.Stream()      # a stream of its own: the fused kernel
 
     def tendency(U):
         u.upload(U)
-        s.get_residual(u.addr, r.addr)
-        s.mult_inv_mass_matrix(dt, r.addr, r.addr)
+        s.get_residual(u.addr, r.addr, st.h.value)
+        s.mult_inv_mass_matrix(dt, r.addr, r.addr, st.h.value)
         hip.synchronize()
         return r.download(U.shape)
 
@@ -84,6 +84,30 @@ def test_step_matches_the_composed_step(order, ne, basis, flux, precision):
         tol = 64 * eps * (2 * order + 1) ** 3 * inc + 4 * 2.0 ** -52 * np.max(np.abs(ref))
         assert np.all(np.isfinite(U1)) and inc > 0.0
         assert d <= tol, (stepper, d, tol, inc)
+
+
+@pytest.mark.parametrize("order,ne,basis,flux", CASES)
+@pytest.mark.parametrize("precision", [None, "FP32"])
+def test_residual_matches_the_fused_kernel(order, ne, basis, flux, precision):
+    """on the handle's stream, against the fused kernel on the caller's"""
+    print(f"two-pass residual p={order} {ne} {basis} {flux} {precision}", flush=True)
+    s, _ = solver(order, ne, basis, flux, "RK4", precision)
+    with s:
+        U = s.get_state()
+        u, ra, rb, st = hip.Buffer.from_array(U), hip.Buffer(U.size), hip.Buffer(U.size), hip.Stream()
+        s.get_residual(u.addr, ra.addr)
+        s.get_residual(u.addr, rb.addr, st.h.value)
+        hip.synchronize()
+        a, b = ra.download(U.shape), rb.download(U.shape)
+        for buf in (u, ra, rb):
+            buf.free()
+    # differences of sums of some hundred rounded operations on flux terms
+    # of at most the states' scale (5) times the largest face
+    h = sorted((hi - lo) / n for lo, hi, n in zip((-5., -4., -3.), (5., 4., 3.), ne))
+    size = 5. * np.max(np.abs(U)) * h[1] * h[2]
+    eps = 2.0 ** -53 if precision is None else 2.0 ** -24
+    assert np.all(np.isfinite(a)) and np.max(np.abs(b)) > 0.0
+    assert np.max(np.abs(a - b)) <= 64 * eps * (np.max(np.abs(b)) + size)
 
 
 @pytest.mark.parametrize("precision", [None, "FP32"])
