@@ -17,6 +17,7 @@
 #include <sstream>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "dg_solver_impl.hpp"
@@ -60,44 +61,11 @@ __device__ inline float from_bf16(uint16_t h) {
 }
 
 __device__ inline float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
-__device__ inline float gelu_d(float z) {
-    return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
-}
-
-// output gradient of the mean squared error in normalised target units:
-// G = 2 (O - Y / yscale) / (M NO); per-block partial sums of the squared error
-__global__ void loss_grad(const float* __restrict__ O, const float* __restrict__ Y,
-                          const float* __restrict__ yscale, float* __restrict__ G, double* __restrict__ part,
-                          long M) {
-    __shared__ double red[TB];
-    const long t = (long)blockIdx.x * TB + threadIdx.x;
-    double e2 = 0.;
-    if (t < M * NO) {
-        const int n = (int)(t % NO);
-        const float d = O[t] - Y[t] / yscale[n];
-        G[t] = 2.0f * d / (float)(M * NO);
-        e2 = (double)d * d;
-    }
-    red[threadIdx.x] = e2;
-    __syncthreads();
-    for (int s = TB / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-// rows idx[i] of X (NF) and Y (NO) into contiguous mini-batch buffers
-__global__ void gather_rows(const float* __restrict__ X, const float* __restrict__ Y, const int* __restrict__ idx,
-                            float* __restrict__ Xb, float* __restrict__ Yb, long B, long nrows) {
-    const long t = (long)blockIdx.x * TB + threadIdx.x;
-    if (t >= B * (NF + NO)) return;
-    const long i = t / (NF + NO);
-    const int c = (int)(t % (NF + NO));
-    long r = idx[i];
-    r = r < 0 ? 0 : (r >= nrows ? nrows - 1 : r);
-    if (c < NF) Xb[i * NF + c] = X[r * NF + c];
-    else Yb[i * NO + (c - NF)] = Y[r * NO + (c - NF)];
+// gelu(z), and its derivative in d
+__device__ inline float gelu_both(float z, float& d) {
+    const float e = 1.0f + erff(z * 0.70710678118654752f);
+    d = 0.5f * e + z * 0.39894228040143268f * expf(-0.5f * z * z);
+    return 0.5f * z * e;
 }
 
 // Gaussian jitter of the mini-batch features, noise standard deviations in
@@ -109,32 +77,12 @@ __device__ inline unsigned long long mix64(unsigned long long z) {
     z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
     return z ^ (z >> 31);
 }
-__global__ void jitter_kernel(float* __restrict__ Xb, const float* __restrict__ scale, float noise, long n,
-                              unsigned long long key) {
-    const long t = (long)blockIdx.x * TB + threadIdx.x;
-    if (t >= n) return;
-    const unsigned long long h = mix64(key ^ mix64((unsigned long long)t));
+__device__ inline float jitter(float noise, float scale, unsigned long long t, unsigned long long key) {
+    const unsigned long long h = mix64(key ^ mix64(t));
     const float u1 = ((float)(h >> 40) + 0.5f) * (1.0f / 16777216.0f);
     const float u2 = ((float)((h >> 16) & 0xffffffu) + 0.5f) * (1.0f / 16777216.0f);
     const float g = sqrtf(-2.0f * logf(u1)) * cosf(6.283185307179586f * u2);
-    Xb[t] += noise * g / scale[t % NF];
-}
-
-// Adam (Kingma & Ba 2015) on the FP32 master parameters; the BF16 working
-// copy follows
-__global__ void adam_step(float* __restrict__ p, uint16_t* __restrict__ pb, const float* __restrict__ g,
-                          float* __restrict__ m1, float* __restrict__ m2, float lr, float b1, float b2, float eps,
-                          float c1, float c2, int n) {
-    const int i = blockIdx.x * TB + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float a = b1 * m1[i] + (1.f - b1) * gi;
-    const float v = b2 * m2[i] + (1.f - b2) * gi * gi;
-    m1[i] = a;
-    m2[i] = v;
-    const float q = p[i] - lr * (a / c1) / (sqrtf(v / c2) + eps);
-    p[i] = q;
-    pb[i] = to_bf16(q);
+    return noise * g / scale;
 }
 
 __global__ void to_bf16_kernel(const float* __restrict__ p, uint16_t* __restrict__ pb, int n) {
@@ -403,177 +351,325 @@ __global__ __launch_bounds__(MT) void mlp_infer_kernel(const float* __restrict__
 // arithmetic is that of a plain FP32 network with bf16 weights up to the
 // order of the FP32 sums.
 // ---------------------------------------------------------------------------
-constexpr int GW = 4;                          // waves per training workgroup
 constexpr int WV = 64;                         // lanes per wave
-constexpr int NJH = 2;                         // 16-column tiles per wave of the 128-wide layers
+constexpr int RT = 16;                         // rows of a train_rows workgroup
+constexpr int RW = NH / 16;                    // its waves: a 16-column tile of the hidden layers each
+constexpr int RB = RW * WV;
+constexpr int GW = 4;                          // waves of a weight-gradient workgroup
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Z[m][n] = sum_k A'[m][k] W[k][n] + b[n] and H = act(Z) (Z kept when
-// non-null), A' = (A - mean) scale when mean is non-null.  Each wave takes
-// 16 rows and NJ 16-column tiles of the N outputs, the tiles of column
-// group blockIdx.y (columns >= N masked).
-template <bool ACT, int NJ>
-__global__ __launch_bounds__(GW * WV) void mfma_fwd(const float* __restrict__ A, const float* __restrict__ mean,
-                                                    const float* __restrict__ scale, const uint16_t* __restrict__ W,
-                                                    const float* __restrict__ b, float* __restrict__ Z,
-                                                    float* __restrict__ H, long M, int K, int N) {
-    const int lane = threadIdx.x & (WV - 1), c = lane & 15, kq = lane >> 4;
-    const long m0 = ((long)blockIdx.x * GW + (threadIdx.x / WV)) * 16;
-    if (m0 >= M) return;                       // whole waves; no barrier follows
-    const long ma = m0 + c;
-    const bool rowok = ma < M;
-    const int n0 = blockIdx.y * 16 * NJ;
-    f32x4 acc[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int n = n0 + 16 * j + c;
-        const float bn = n < N ? b[n] : 0.f;
-        acc[j] = f32x4{bn, bn, bn, bn};
+// The bf16 weights in the order of train_rows' lanes: for each 16-column tile
+// of a layer's outputs, 16 bytes per lane of the weights of eight MFMA steps;
+// forward W1, W2, W3, then W3 and W2 for the backward steps (rows as
+// columns).  17 16-byte loads per lane in place of 124 2-byte ones.
+constexpr int ST1 = (NF + 3) / 4, ST2 = NH / 4, ST3 = NO / 4;      // MFMA steps over the layers' inputs
+constexpr int S1 = (ST1 + 7) / 8, S2 = (ST2 + 7) / 8, S3 = (ST3 + 7) / 8;
+constexpr int TG = WV * 8;                     // weights of one tile and eight steps
+constexpr int LI1 = 0, LI2 = LI1 + RW * S1 * TG, LI3 = LI2 + RW * S2 * TG, LB3 = LI3 + (NO + 15) / 16 * S2 * TG,
+              LB2 = LB3 + RW * S3 * TG, LANE_IMG = LB2 + RW * S2 * TG;
+__device__ __forceinline__ int lane_slot(int img, int groups, int k, int n) {   // input k, output n
+    return img + ((n / 16 * groups + k / 32) * WV + (k & 3) * 16 + (n & 15)) * 8 + (k / 4 & 7);
+}
+__device__ __forceinline__ void store_lane_weights(uint16_t* img, int i, uint16_t v) {
+    if (i < OFF_B1) {
+        img[lane_slot(LI1, S1, i / NH, i % NH)] = v;
+    } else if (i >= OFF_W2 && i < OFF_B2) {
+        const int k = (i - OFF_W2) / NH, n = (i - OFF_W2) % NH;
+        img[lane_slot(LI2, S2, k, n)] = v;
+        img[lane_slot(LB2, S2, n, k)] = v;
+    } else if (i >= OFF_W3 && i < OFF_B3) {
+        const int k = (i - OFF_W3) / NO, n = (i - OFF_W3) % NO;
+        img[lane_slot(LI3, S2, k, n)] = v;
+        img[lane_slot(LB3, S3, n, k)] = v;
     }
-    for (int k0 = 0; k0 < K; k0 += 4) {
-        const int k = k0 + kq;
+}
+__global__ void pack_lane_weights(const uint16_t* __restrict__ pb, uint16_t* __restrict__ img) {
+    const int i = blockIdx.x * TB + threadIdx.x;
+    if (i < NP) store_lane_weights(img, i, pb[i]);
+}
+// x is in its register here: what follows does not wait for its load (nor,
+// the counter of loads and stores being one, for stores issued in between)
+template <class T>
+__device__ __forceinline__ void arrived(T& x) {
+    asm volatile("" : "+v"(x));
+}
+template <int S>
+struct LaneWeights {
+    uint4 v[S];
+    __device__ __forceinline__ void arrive() {
+#pragma unroll
+        for (int g = 0; g < S; ++g) {
+            arrived(v[g].x);
+            arrived(v[g].y);
+            arrived(v[g].z);
+            arrived(v[g].w);
+        }
+    }
+    __device__ __forceinline__ void load(const uint16_t* img, int tile, int lane) {
+#pragma unroll
+        for (int g = 0; g < S; ++g) v[g] = *reinterpret_cast<const uint4*>(img + ((tile * S + g) * WV + lane) * 8);
+    }
+    __device__ __forceinline__ float operator[](int i) const {
+        const uint4& q = v[i / 8];
+        const int h = i % 8 / 2;
+        const uint32_t x = h == 0 ? q.x : (h == 1 ? q.y : (h == 2 ? q.z : q.w));
+        const uint32_t u = i & 1 ? x & 0xffff0000u : x << 16;
+        float f;
+        std::memcpy(&f, &u, 4);
+        return f;
+    }
+};
+
+// Position of a workgroup in the launch's sequence: the grid is a multiple
+// of 8, workgroups go round the 8 XCDs, and each XCD walks a contiguous
+// eighth, so that train_wgrad finds the rows of its chunks in its own L2.
+__device__ __forceinline__ unsigned xcd_walk() {
+    return (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+}
+
+// Forward pass, loss and the gradients of the layer outputs for 16 rows of a
+// mini-batch: gathered (rows idx, or row m itself for null), jittered and
+// normalised rows Xn, activations H1 and H2, gradients G3 (mean squared error
+// in normalised target units, 2 (O - Y / yscale) / (M NO)), G2 and G1, and
+// the rows' sum of squared errors in part.  A wave keeps the pre-activations
+// of its column tile in registers from the forward to the backward pass, the
+// layers meet in LDS (row strides 4 modulo 64 banks and 4 rows x 16 columns
+// per access: no conflicts), and all weights are on their way to registers
+// while the rows are gathered.
+// Bound: latency and issue of the two waves per SIMD that 4096 rows are (256
+// workgroups): some 2000 instructions a wave, many of them the error function,
+// and 124 dependent MFMAs behind the gather.  4096 rows take 13.6 us (26 with
+// 2-byte weight loads); one launch in place of the eight of gather, jitter,
+// three forward layers, loss and two backward ones.  A mini-batch of 4096
+// with its parameter update: 118 us in 13 launches before, 33 in 3.
+struct TrainRows {
+    const float *X, *Y, *xs, *p;
+    const uint16_t* img;             // lane_slot's order
+    const int* idx;
+    long nrows, M;
+    float noise;
+    unsigned long long key;
+    float *Xn, *H1, *H2, *G1, *G2, *G3;
+    double* part;
+};
+
+__global__ __launch_bounds__(RB) void train_rows(TrainRows A) {
+    constexpr int SX = 76, SH = NH + 4, SO = 44;
+    static_assert(NO % 4 == 0 && 4 * ST1 <= SX && NO <= SO, "LDS rows");
+    __shared__ float xn[RT * SX], h1[RT * SH], h2[RT * SH], g2[RT * SH], g3[RT * SO];
+    __shared__ long row[RT];
+    __shared__ double red[RW];
+    const int tid = threadIdx.x, w = tid / WV, lane = tid & (WV - 1), c = lane & 15, kq = lane >> 4;
+    const int n = 16 * w + c, no = n < NO ? n : 0;
+    const long r0 = (long)xcd_walk() * RT;
+    if (r0 >= A.M) return;
+    LaneWeights<S1> w1;
+    LaneWeights<S2> w2, w3, t2;
+    LaneWeights<S3> t3;
+    w1.load(A.img + LI1, w, lane);
+    w2.load(A.img + LI2, w, lane);
+    w3.load(A.img + LI3, 16 * w < NO ? w : 0, lane);
+    t3.load(A.img + LB3, w, lane);
+    t2.load(A.img + LB2, w, lane);
+    float b1 = A.p[OFF_B1 + n], b2 = A.p[OFF_B2 + n], b3 = A.p[OFF_B3 + no], ys = A.xs[2 * NF + no];
+    if (tid < RT) {
+        const long m = r0 + tid < A.M ? r0 + tid : A.M - 1;
+        long r = m;
+        if (A.idx) {
+            r = A.idx[m];
+            r = r < 0 ? 0 : (r >= A.nrows ? A.nrows - 1 : r);
+        }
+        row[tid] = r;
+    }
+    __syncthreads();
+    float y[4];                                // targets of the output tile, in flight over the layers
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[r] = A.Y[row[4 * kq + r] * NO + no];
+    for (int t = tid; t < RT * SX; t += RB) {
+        const int q = t / SX, k = t - q * SX;
+        const long m = r0 + q;
         float a = 0.f;
-        if (rowok && k < K) {
-            a = A[ma * K + k];
-            if (mean) a = (a - mean[k]) * scale[k];
+        if (k < NF && m < A.M) {
+            a = A.X[row[q] * NF + k];
+            if (A.noise > 0.f) a += jitter(A.noise, A.xs[NF + k], (unsigned long long)(m * NF + k), A.key);
+            a = (a - A.xs[k]) * A.xs[NF + k];
+            A.Xn[m * NF + k] = a;
         }
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int n = n0 + 16 * j + c;
-            const float w = (k < K && n < N) ? from_bf16(W[(size_t)k * N + n]) : 0.f;
-            acc[j] = mfma4(a, w, acc[j]);
-        }
+        xn[t] = a;
     }
+    w1.arrive();
+    w2.arrive();
+    w3.arrive();
+    t3.arrive();
+    t2.arrive();
+    for (float& v : y) arrived(v);
+    arrived(b1);
+    arrived(b2);
+    arrived(b3);
+    arrived(ys);
+    __syncthreads();
+    auto layer = [&](const float* in, int stride, const auto& wt, auto steps, f32x4 acc) {
+        constexpr int K = decltype(steps)::value;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int n = n0 + 16 * j + c;
+        for (int i = 0; i < K; ++i) acc = mfma4(in[c * stride + 4 * i + kq], wt[i], acc);
+        return acc;
+    };
+    auto bias = [](float b) { return f32x4{b, b, b, b}; };
+    // the tile to LDS and to memory (whose arrays hold whole tiles of rows)
+    auto put = [&](float* o, int stride, float* out, int width, int r, float v) {
+        o[(4 * kq + r) * stride + n] = v;
+        out[(r0 + 4 * kq) * width + n + r * width] = v;
+    };
+    float dz1[4], dz2[4];
+    const f32x4 z1 = layer(xn, SX, w1, std::integral_constant<int, ST1>(), bias(b1));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) put(h1, SH, A.H1, NH, r, gelu_both(z1[r], dz1[r]));
+    __syncthreads();
+    const f32x4 z2 = layer(h1, SH, w2, std::integral_constant<int, ST2>(), bias(b2));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) put(h2, SH, A.H2, NH, r, gelu_both(z2[r], dz2[r]));
+    __syncthreads();
+    double e2 = 0.;
+    if (16 * w < NO) {
+        const f32x4 o = layer(h2, SH, w3, std::integral_constant<int, ST2>(), bias(b3));
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const long m = m0 + 4 * kq + r;
-            if (m < M && n < N) {
-                const float z = acc[j][r];
-                if (Z) Z[m * N + n] = z;
-                H[m * N + n] = ACT ? gelu(z) : z;
+            const int q = 4 * kq + r;
+            const float d = r0 + q < A.M ? o[r] - y[r] / ys : 0.f;
+            if (n < NO) {
+                put(g3, SO, A.G3, NO, r, 2.0f * d / (float)(A.M * NO));
+                e2 += (double)d * d;
             }
         }
     }
-}
-
-// Gin[m][k] = (sum_n G[m][n] W[k][n]) gelu'(Z[m][k]) for the KO inputs k
-// of a layer with N outputs; each wave takes 16 rows and the NJ 16-column
-// tiles of column group blockIdx.y
-template <int KO, int NJ>
-__global__ __launch_bounds__(GW * WV) void mfma_bwd_in(const float* __restrict__ G, const uint16_t* __restrict__ W,
-                                                       const float* __restrict__ Z, float* __restrict__ Gin, long M,
-                                                       int N) {
-    static_assert(KO % (16 * NJ) == 0, "whole column groups");
-    const int lane = threadIdx.x & (WV - 1), c = lane & 15, kq = lane >> 4;
-    const int k0 = blockIdx.y * 16 * NJ;
-    const long m0 = ((long)blockIdx.x * GW + (threadIdx.x / WV)) * 16;
-    if (m0 >= M) return;
-    const long ma = m0 + c;
-    const bool rowok = ma < M;
-    f32x4 acc[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int n0 = 0; n0 < N; n0 += 4) {
-        const int n = n0 + kq;
-        const float g = (rowok && n < N) ? G[ma * N + n] : 0.f;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int k = k0 + 16 * j + c;
-            const float w = n < N ? from_bf16(W[(size_t)k * N + n]) : 0.f;
-            acc[j] = mfma4(g, w, acc[j]);
-        }
+    for (int off = WV / 2; off > 0; off >>= 1) e2 += __shfl_down(e2, off, WV);
+    if (lane == 0) red[w] = e2;
+    __syncthreads();
+    if (tid == 0) {
+        double v = 0.;
+        for (int i = 0; i < RW; ++i) v += red[i];
+        A.part[r0 / RT] = v;
     }
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const f32x4 d2 = layer(g3, SO, t3, std::integral_constant<int, ST3>(), zero);
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int k = k0 + 16 * j + c;
+    for (int r = 0; r < 4; ++r) put(g2, SH, A.G2, NH, r, d2[r] * dz2[r]);
+    __syncthreads();
+    const f32x4 d1 = layer(g2, SH, t2, std::integral_constant<int, ST2>(), zero);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const long m = m0 + 4 * kq + r;
-            if (m < M) Gin[m * KO + k] = acc[j][r] * gelu_d(Z[m * KO + k]);
-        }
-    }
+    for (int r = 0; r < 4; ++r) A.G1[(r0 + 4 * kq) * NH + n + r * NH] = d1[r] * dz1[r];
 }
 
 // Weight and bias gradients of a layer with K inputs and N outputs, partial
-// over one chunk of rows: part[s][k][n] = sum_{m in chunk s} A'[m][k]
-// G[m][n], with the row k = K the bias (A' = 1); A' normalised as in
-// mfma_fwd when mean is non-null.  Workgroup (16-row k tile, chunk s,
-// column group of NJ 16-column tiles; columns >= N masked); its waves split
-// the chunk's rows and add their tiles in LDS, in a fixed order.
-template <int NJ>
-__global__ __launch_bounds__(GW * WV) void mfma_wgrad(const float* __restrict__ A, const float* __restrict__ mean,
-                                                      const float* __restrict__ scale, const float* __restrict__ G,
-                                                      float* __restrict__ part, long M, int K, int N, long chunk) {
-    __shared__ f32x4 red[GW][NJ][WV];
+// over one chunk of rows: part[k][n] = sum_{m in [mb, me)} A[m][k] G[m][n],
+// with the row k = K the bias (A = 1), for the 16 rows k0 .. of the layer and
+// all its columns.  The waves split the chunk's rows and add their tiles in
+// LDS, in a fixed order.  A lane reads four neighbouring columns at once:
+// tile j of a group of four holds the columns 4 c + j.  Bound: latency (4096
+// rows: 64 MFMAs per wave, 8.8 us for the three layers).
+template <int K, int N>
+__device__ __forceinline__ void wgrad_tile(const float* __restrict__ A, const float* __restrict__ G,
+                                           float* __restrict__ part, int k0, long mb, long me, f32x4* red) {
+    constexpr int NG = (N + 63) / 64, NJ = 4 * NG;
     const int wv = threadIdx.x / WV, lane = threadIdx.x & (WV - 1), c = lane & 15, kq = lane >> 4;
-    const int k0 = blockIdx.x * 16, k = k0 + c, n0 = blockIdx.z * 16 * NJ;
-    const long mb = (long)blockIdx.y * chunk, me = mb + chunk < M ? mb + chunk : M;
+    const int k = k0 + c;
     f32x4 acc[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
     for (long m4 = mb + 4 * wv; m4 < me; m4 += 4 * GW) {
         const long m = m4 + kq;
-        const bool ok = m < me;
-        float a = 0.f;
-        if (ok && k <= K) {
-            if (k == K) {
-                a = 1.f;
-            } else {
-                a = A[m * K + k];
-                if (mean) a = (a - mean[k]) * scale[k];
-            }
-        }
+        const bool ok = m < me;                // all rows but the last ones of the batch's last chunk
+        const long mc = ok ? m : mb;
+        float a = A[mc * K + (k < K ? k : 0)];
+        a = ok ? (k < K ? a : (k == K ? 1.f : 0.f)) : 0.f;
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int n = n0 + 16 * j + c;
-            const float g = (ok && n < N) ? G[m * N + n] : 0.f;
-            acc[j] = mfma4(a, g, acc[j]);
+        for (int q = 0; q < NG; ++q) {
+            const int n = 64 * q + 4 * c;      // the columns past N are not stored
+            f32x4 g = *reinterpret_cast<const f32x4*>(G + mc * N + (n < N ? n : 0));
+            if (m4 + 4 > me && !ok) g = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[4 * q + j] = mfma4(a, g[j], acc[4 * q + j]);
         }
     }
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) red[wv][j][lane] = acc[j];
+    for (int j = 0; j < NJ; ++j) red[(wv * NJ + j) * WV + lane] = acc[j];
     __syncthreads();
-    for (int i = threadIdx.x; i < NJ * WV; i += GW * WV) {
-        const int j = i / WV, l = i % WV;
-        f32x4 v = red[0][j][l];
+    for (int i = threadIdx.x; i < NG * WV; i += GW * WV) {
+        const int q = i / WV, l = i % WV, n = 64 * q + 4 * (l & 15);
+        if (n >= N) continue;
+        f32x4 v[4];
 #pragma unroll
-        for (int w = 1; w < GW; ++w) v += red[w][j][l];
-        const int n = n0 + 16 * j + (l & 15);
+        for (int j = 0; j < 4; ++j) {
+            v[j] = red[(4 * q + j) * WV + l];
+#pragma unroll
+            for (int w = 1; w < GW; ++w) v[j] += red[(w * NJ + 4 * q + j) * WV + l];
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int kk = k0 + 4 * (l >> 4) + r;
-            if (kk <= K && n < N) part[(size_t)blockIdx.y * NP + (size_t)kk * N + n] = v[r];
+            if (kk <= K) *reinterpret_cast<f32x4*>(part + kk * N + n) = f32x4{v[0][r], v[1][r], v[2][r], v[3][r]};
         }
     }
 }
 
-// g[i] = sum_s part[s][i] over the row chunks (fixed order)
-__global__ void grad_reduce(const float* __restrict__ part, float* __restrict__ g, int nchunk) {
-    const int i = blockIdx.x * TB + threadIdx.x;
-    if (i >= NP) return;
-    float v = 0.f;
-    for (int s = 0; s < nchunk; ++s) v += part[(size_t)s * NP + i];
-    g[i] = v;
+// All three layers in one launch: workgroup (16-row k tile of a layer, chunk)
+constexpr int KT1 = (NF + 16) / 16, KT2 = (NH + 16) / 16;      // k tiles with the bias row
+static_assert(NH % 64 == 0 && NO % 4 == 0 && OFF_W2 % 4 == 0 && OFF_W3 % 4 == 0 && NP % 4 == 0,
+              "16-byte groups of columns");
+__global__ __launch_bounds__(GW * WV) void train_wgrad(TrainRows A, float* __restrict__ gpart, long chunk) {
+    __shared__ f32x4 red[GW * (NH / 16) * WV];
+    const unsigned u = xcd_walk(), s = u / (KT1 + 2 * KT2);
+    const int t = (int)(u - s * (KT1 + 2 * KT2));
+    const long mb = (long)s * chunk, me = mb + chunk < A.M ? mb + chunk : A.M;
+    if (mb >= A.M) return;
+    float* part = gpart + (size_t)s * NP;
+    if (t < KT2) wgrad_tile<NH, NH>(A.H1, A.G2, part + OFF_W2, 16 * t, mb, me, red);
+    else if (t < KT2 + KT1) wgrad_tile<NF, NH>(A.Xn, A.G1, part + OFF_W1, 16 * (t - KT2), mb, me, red);
+    else wgrad_tile<NH, NO>(A.H2, A.G3, part + OFF_W3, 16 * (t - KT2 - KT1), mb, me, red);
 }
 
-// acc += (sum of the nb partial squared errors) * inv, one block, fixed order
-__global__ void loss_add(const double* __restrict__ part, long nb, double inv, double* __restrict__ acc) {
-    __shared__ double red[TB];
-    double v = 0.;
-    for (long i = threadIdx.x; i < nb; i += TB) v += part[i];
-    red[threadIdx.x] = v;
-    __syncthreads();
-    for (int s = TB / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
+// g[i] = sum_s part[s][i] over the row chunks (fixed order), with ADAM then
+// the Adam update (Kingma & Ba 2015) of the FP32 master parameters and their
+// BF16 working copy; the last workgroup adds the rows' squared errors
+// (nb partial sums) times inv to the loss, in a fixed order.
+struct AdamStep {
+    float *p, *m1, *m2;
+    uint16_t *pb, *img;
+    float lr, b1, b2, eps, c1, c2;
+};
+template <bool ADAM>
+__global__ __launch_bounds__(WV) void train_update(const float* __restrict__ part, float* __restrict__ g, int nchunk,
+                                                   AdamStep S, const double* __restrict__ e2, long nb, double inv,
+                                                   double* __restrict__ loss) {
+    if (blockIdx.x == gridDim.x - 1) {
+        double v = 0.;
+        for (long i = threadIdx.x; i < nb; i += WV) v += e2[i];
+        for (int off = WV / 2; off > 0; off >>= 1) v += __shfl_down(v, off, WV);
+        if (threadIdx.x == 0) loss[0] += v * inv;
+        return;
     }
-    if (threadIdx.x == 0) acc[0] += red[0] * inv;
+    const int i = blockIdx.x * WV + threadIdx.x;
+    if (i >= NP) return;
+    float v = 0.f;
+#pragma unroll 8
+    for (int s = 0; s < nchunk; ++s) v += part[(size_t)s * NP + i];
+    if constexpr (ADAM) {
+        const float a = S.b1 * S.m1[i] + (1.f - S.b1) * v;
+        const float q2 = S.b2 * S.m2[i] + (1.f - S.b2) * v * v;
+        S.m1[i] = a;
+        S.m2[i] = q2;
+        const float q = S.p[i] - S.lr * (a / S.c1) / (sqrtf(q2 / S.c2) + S.eps);
+        S.p[i] = q;
+        const uint16_t h = to_bf16(q);
+        S.pb[i] = h;
+        store_lane_weights(S.img, i, h);
+    } else {
+        g[i] = v;
+    }
 }
 
 __global__ void clear_f64_kernel(double* p) { p[threadIdx.x] = 0.; }
@@ -623,14 +719,14 @@ struct dg_mlp {
     float* p = nullptr;          // master parameters [NP]
     uint16_t* pb = nullptr;      // BF16 working copy
     uint16_t* img = nullptr;     // the inference kernel's LDS image of the bf16 weights
+    uint16_t* lane_img = nullptr;   // the training kernels' copy (lane_slot)
     bool img_stale = true;       // pb changed since img was built
     float* g = nullptr;          // gradient
     float* m1 = nullptr;         // Adam moments
     float* m2 = nullptr;
     float* xs = nullptr;         // feature mean [NF], scale [NF], target scale [NO]
     long cap = 0;                // rows the activation buffers hold
-    float *Z1 = nullptr, *H1 = nullptr, *Z2 = nullptr, *H2 = nullptr, *O = nullptr, *G3 = nullptr,
-          *G2 = nullptr, *G1 = nullptr, *Xb = nullptr, *Yb = nullptr;
+    float *Xn = nullptr, *H1 = nullptr, *H2 = nullptr, *G3 = nullptr, *G2 = nullptr, *G1 = nullptr;
     double* part = nullptr;
     float* gpart = nullptr;      // per-chunk weight-gradient partials [GCHUNKS][NP]
     double* lacc = nullptr;      // training loss accumulator (device)
@@ -641,12 +737,12 @@ struct dg_mlp {
 namespace {
 
 void free_acts(dg_mlp* m) {
-    for (float* q : {m->Z1, m->H1, m->Z2, m->H2, m->O, m->G3, m->G2, m->G1, m->Xb, m->Yb})
+    for (float* q : {m->Xn, m->H1, m->H2, m->G3, m->G2, m->G1})
         if (q) (void)hipFree(q);
     if (m->part) (void)hipFree(m->part);
     if (m->gpart) (void)hipFree(m->gpart);
     if (m->lacc) (void)hipFree(m->lacc);
-    m->Z1 = m->H1 = m->Z2 = m->H2 = m->O = m->G3 = m->G2 = m->G1 = m->Xb = m->Yb = nullptr;
+    m->Xn = m->H1 = m->H2 = m->G3 = m->G2 = m->G1 = nullptr;
     m->part = nullptr;
     m->gpart = nullptr;
     m->lacc = nullptr;
@@ -670,20 +766,17 @@ void launch_infer(dg_mlp* m, const float* X, float* C, double bound, long rows, 
 }
 
 void ensure_acts(dg_mlp* m, long rows) {
+    rows = (rows + RT - 1) / RT * RT;          // train_rows writes whole tiles
     if (rows <= m->cap) return;
     free_acts(m);
     auto al = [&](float** q, long n) { hcheck(hipMalloc(q, (size_t)n * sizeof(float)), "hipMalloc(mlp)"); };
-    al(&m->Z1, rows * NH);
     al(&m->H1, rows * NH);
-    al(&m->Z2, rows * NH);
     al(&m->H2, rows * NH);
-    al(&m->O, rows * NO);
     al(&m->G3, rows * NO);
     al(&m->G2, rows * NH);
     al(&m->G1, rows * NH);
-    al(&m->Xb, rows * NF);
-    al(&m->Yb, rows * NO);
-    hcheck(hipMalloc(&m->part, (size_t)nblk(rows * NO) * sizeof(double)), "hipMalloc(mlp)");
+    al(&m->Xn, rows * NF);
+    hcheck(hipMalloc(&m->part, (size_t)((rows + RT - 1) / RT) * sizeof(double)), "hipMalloc(mlp)");
     hcheck(hipMalloc(&m->gpart, (size_t)GCHUNKS * NP * sizeof(float)), "hipMalloc(mlp)");
     hcheck(hipMalloc(&m->lacc, sizeof(double)), "hipMalloc(mlp)");
     m->cap = rows;
@@ -696,46 +789,51 @@ long grad_chunk(long M) {
     return c < 64 ? 64 : c;
 }
 
-// forward pass of rows X (raw features) into m->O (normalised outputs)
-void forward(dg_mlp* m, const float* X, long rows) {
-    hipStream_t st = m->stream;
-    const float* mean = m->xs;
-    const float* scale = m->xs + NF;
-    const unsigned rt = (unsigned)((rows + 16 * GW - 1) / (16 * GW));
-    const dim3 gh(rt, NH / (16 * NJH)), go(rt, (NO + 15) / 16), block(GW * WV);
-    hipLaunchKernelGGL((mfma_fwd<true, NJH>), gh, block, 0, st, X, mean, scale, m->pb + OFF_W1, m->p + OFF_B1,
-                       m->Z1, m->H1, rows, NF, NH);
-    hipLaunchKernelGGL((mfma_fwd<true, NJH>), gh, block, 0, st, m->H1, nullptr, nullptr, m->pb + OFF_W2,
-                       m->p + OFF_B2, m->Z2, m->H2, rows, NH, NH);
-    hipLaunchKernelGGL((mfma_fwd<false, 1>), go, block, 0, st, m->H2, nullptr, nullptr,
-                       m->pb + OFF_W3, m->p + OFF_B3, nullptr, m->O, rows, NH, NO);
-    hcheck(hipGetLastError(), "mlp forward");
+// the training kernels' copy of the bf16 weights, before a run of mini-batches
+// (train_update keeps it from one to the next)
+void pack_lanes(dg_mlp* m) {
+    hipLaunchKernelGGL(pack_lane_weights, dim3(nblk(NP)), dim3(TB), 0, m->stream, m->pb, m->lane_img);
+    hcheck(hipGetLastError(), "weight copy kernel");
 }
 
-// loss and gradient (into m->g) of rows X, Y: the batch's mean squared
-// error is added to m->lacc on the device (no host synchronisation)
-void backward(dg_mlp* m, const float* X, const float* Y, long rows) {
+// Loss and gradient of a mini-batch of M rows: the batch's mean squared error
+// is added to m->lacc on the device (no host synchronisation); the gradient
+// goes into m->g, or with adam straight into the parameters.
+void mini_batch(dg_mlp* m, const float* X, const float* Y, const int* idx, long nrows, long M, float noise,
+                const AdamStep* adam) {
     hipStream_t st = m->stream;
-    const float* mean = m->xs;
-    const float* scale = m->xs + NF;
-    const float* ys = m->xs + 2 * NF;
-    forward(m, X, rows);
-    const unsigned nb = nblk(rows * NO);
-    hipLaunchKernelGGL(loss_grad, dim3(nb), dim3(TB), 0, st, m->O, Y, ys, m->G3, m->part, rows);
-    hipLaunchKernelGGL(loss_add, dim3(1), dim3(TB), 0, st, m->part, (long)nb, 1.0 / (double)(rows * NO), m->lacc);
-    const long chunk = grad_chunk(rows);
-    const unsigned nch = (unsigned)((rows + chunk - 1) / chunk);
-    const dim3 gh((unsigned)((rows + 16 * GW - 1) / (16 * GW)), NH / (16 * NJH)), block(GW * WV);
-    hipLaunchKernelGGL((mfma_wgrad<1>), dim3((NH + 1 + 15) / 16, nch, (NO + 15) / 16), block, 0, st, m->H2,
-                       nullptr, nullptr, m->G3, m->gpart + OFF_W3, rows, NH, NO, chunk);
-    hipLaunchKernelGGL((mfma_bwd_in<NH, NJH>), gh, block, 0, st, m->G3, m->pb + OFF_W3, m->Z2, m->G2, rows, NO);
-    hipLaunchKernelGGL((mfma_wgrad<NJH>), dim3((NH + 1 + 15) / 16, nch, NH / (16 * NJH)), block, 0, st, m->H1,
-                       nullptr, nullptr, m->G2, m->gpart + OFF_W2, rows, NH, NH, chunk);
-    hipLaunchKernelGGL((mfma_bwd_in<NH, NJH>), gh, block, 0, st, m->G2, m->pb + OFF_W2, m->Z1, m->G1, rows, NH);
-    hipLaunchKernelGGL((mfma_wgrad<NJH>), dim3((NF + 1 + 15) / 16, nch, NH / (16 * NJH)), block, 0, st, X, mean,
-                       scale, m->G1, m->gpart + OFF_W1, rows, NF, NH, chunk);
-    hipLaunchKernelGGL(grad_reduce, dim3(nblk(NP)), dim3(TB), 0, st, m->gpart, m->g, (int)nch);
-    hcheck(hipGetLastError(), "mlp backward");
+    TrainRows A;
+    A.X = X;
+    A.Y = Y;
+    A.xs = m->xs;
+    A.p = m->p;
+    A.img = m->lane_img;
+    A.idx = idx;
+    A.nrows = nrows;
+    A.M = M;
+    A.noise = noise;
+    A.key = (unsigned long long)m->step * 0x100000001ull;
+    A.Xn = m->Xn;
+    A.H1 = m->H1;
+    A.H2 = m->H2;
+    A.G1 = m->G1;
+    A.G2 = m->G2;
+    A.G3 = m->G3;
+    A.part = m->part;
+    const unsigned nr = (unsigned)((M + RT - 1) / RT);
+    hipLaunchKernelGGL(train_rows, dim3((nr + 7u) & ~7u), dim3(RB), 0, st, A);
+    const long chunk = grad_chunk(M);
+    const unsigned nch = (unsigned)((M + chunk - 1) / chunk);
+    hipLaunchKernelGGL(train_wgrad, dim3((nch * (KT1 + 2 * KT2) + 7u) & ~7u), dim3(GW * WV), 0, st, A, m->gpart, chunk);
+    const dim3 ug((NP + WV - 1) / WV + 1);
+    const double inv = 1.0 / (double)(M * NO);
+    if (adam)
+        hipLaunchKernelGGL((train_update<true>), ug, dim3(WV), 0, st, m->gpart, m->g, (int)nch, *adam, m->part,
+                           (long)nr, inv, m->lacc);
+    else
+        hipLaunchKernelGGL((train_update<false>), ug, dim3(WV), 0, st, m->gpart, m->g, (int)nch, AdamStep{}, m->part,
+                           (long)nr, inv, m->lacc);
+    hcheck(hipGetLastError(), "mlp training kernels");
 }
 
 // m->lacc = 0 (a kernel: no memset node on a captured stream)
@@ -885,6 +983,8 @@ int dg_mlp_create(unsigned long long seed, dg_mlp** out) {
         hcheck(hipMalloc(&m->p, NP * sizeof(float)), "hipMalloc(mlp)");
         hcheck(hipMalloc(&m->pb, NP * sizeof(uint16_t)), "hipMalloc(mlp)");
         hcheck(hipMalloc(&m->img, IMG * sizeof(uint16_t)), "hipMalloc(mlp)");
+        hcheck(hipMalloc(&m->lane_img, LANE_IMG * sizeof(uint16_t)), "hipMalloc(mlp)");
+        hcheck(dg::launch_zero(m->lane_img, LANE_IMG * sizeof(uint16_t), m->stream), "zero kernel");   // the padding
         hcheck(hipMalloc(&m->g, NP * sizeof(float)), "hipMalloc(mlp)");
         hcheck(hipMalloc(&m->m1, NP * sizeof(float)), "hipMalloc(mlp)");
         hcheck(hipMalloc(&m->m2, NP * sizeof(float)), "hipMalloc(mlp)");
@@ -926,6 +1026,7 @@ int dg_mlp_destroy(dg_mlp* m) {
         if (q) (void)hipFree(q);
     if (m->pb) (void)hipFree(m->pb);
     if (m->img) (void)hipFree(m->img);
+    if (m->lane_img) (void)hipFree(m->lane_img);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
     return DG_OK;
@@ -1003,7 +1104,8 @@ int dg_mlp_gradient(dg_mlp* m, const float* X_dev, const float* Y_dev, long rows
         hcheck(hipSetDevice(m->device), "hipSetDevice");
         ensure_acts(m, rows);
         clear_loss(m);
-        backward(m, X_dev, Y_dev, rows);
+        pack_lanes(m);
+        mini_batch(m, X_dev, Y_dev, nullptr, rows, rows, 0.f, nullptr);
         const double l = read_loss(m);
         if (loss) *loss = l;
         if (grad_host) hcheck(hipMemcpy(grad_host, m->g, NP * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy");
@@ -1022,22 +1124,15 @@ int dg_mlp_train(dg_mlp* m, const float* X_dev, const float* Y_dev, long nrows, 
         hcheck(hipSetDevice(m->device), "hipSetDevice");
         ensure_acts(m, batch);
         clear_loss(m);
+        pack_lanes(m);
         long nb = 0;
         for (long i0 = 0; i0 + batch <= nidx; i0 += batch) {
-            hipLaunchKernelGGL(gather_rows, dim3(nblk((long)batch * (NF + NO))), dim3(TB), 0, m->stream, X_dev,
-                               Y_dev, idx_dev + i0, m->Xb, m->Yb, (long)batch, nrows);
-            if (noise > 0.f)
-                hipLaunchKernelGGL(jitter_kernel, dim3(nblk((long)batch * NF)), dim3(TB), 0, m->stream, m->Xb,
-                                   m->xs + NF, noise, (long)batch * NF, (unsigned long long)m->step * 0x100000001ull);
-            backward(m, m->Xb, m->Yb, batch);
+            const float b1 = 0.9f, b2 = 0.999f, k = (float)(m->step + 1);
+            const AdamStep adam{m->p, m->m1, m->m2, m->pb, m->lane_img, lr, b1, b2, 1e-8f, 1.f - std::pow(b1, k), 1.f - std::pow(b2, k)};
+            m->img_stale = true;
+            mini_batch(m, X_dev, Y_dev, idx_dev + i0, nrows, batch, noise, &adam);
             ++nb;
             ++m->step;
-            const float b1 = 0.9f, b2 = 0.999f;
-            const float c1 = 1.f - std::pow(b1, (float)m->step), c2 = 1.f - std::pow(b2, (float)m->step);
-            m->img_stale = true;
-            hipLaunchKernelGGL(adam_step, dim3(nblk(NP)), dim3(TB), 0, m->stream, m->p, m->pb, m->g, m->m1, m->m2, lr,
-                               b1, b2, 1e-8f, c1, c2, NP);
-            hcheck(hipGetLastError(), "adam");
         }
         const double sum = read_loss(m);
         if (mean_loss) *mean_loss = nb ? sum / nb : 0.;
