@@ -579,7 +579,6 @@ __device__ __forceinline__ void wgrad_tile(const float* __restrict__ A, const fl
     f32x4 acc[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
     for (long m4 = mb + 4 * wv; m4 < me; m4 += 4 * GW) {
         const long m = m4 + kq;
         const bool ok = m < me;                // all rows but the last ones of the batch's last chunk

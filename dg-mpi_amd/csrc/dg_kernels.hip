@@ -3296,14 +3296,39 @@ constexpr int team_of(int variant) {
     default: return hipErrorInvalidValue;              \
     }
 
+// The launchers are compiled in four objects side by side (Makefile): 1 the
+// fused 3D stage, 2 its batched form, 3 the two passes, 0 the rest.
+hipError_t launch_stage_3d(int P, int flux, const StageArgs& a, const KTables* t, const KGeom& g, hipStream_t st);
+
+#if DG_PART == 1
+hipError_t launch_stage_3d(int P, int flux, const StageArgs& a, const KTables* t, const KGeom& g, hipStream_t st) {
+    DG_DISPATCH_P(P, return stage_p<PP>(flux, a, t, g, st));
+    return hipSuccess;
+}
+
+hipError_t launch_stage_corrected(int P, int flux, const StageArgs& a, const float* C, const KTables* t,
+                                  const KGeom& g, hipStream_t st) {
+    if (P != 1 || g.dim != 3 || g.mapped || g.fp32 || a.mode == MODE_RESIDUAL) return hipErrorInvalidValue;
+    dim3 grid(g.E), block(stage_team<1>());
+    switch (flux) {
+    case 0: hipLaunchKernelGGL((stage_corr_kernel<1, 0>), grid, block, 0, st, a, t, g, C); break;
+    case 1: hipLaunchKernelGGL((stage_corr_kernel<1, 1>), grid, block, 0, st, a, t, g, C); break;
+    default: hipLaunchKernelGGL((stage_corr_kernel<1, 2>), grid, block, 0, st, a, t, g, C); break;
+    }
+    return hipGetLastError();
+}
+
+#elif DG_PART == 0
 hipError_t launch_stage(int P, int flux, const StageArgs& a, const KTables* t, const KGeom& g,
                         hipStream_t st) {
     if (g.dim == 2) {
         DG_DISPATCH_P(P, return stage2d_p<PP>(flux, a, t, g, st));
     }
-    DG_DISPATCH_P(P, return stage_p<PP>(flux, a, t, g, st));
-    return hipSuccess;
+    return launch_stage_3d(P, flux, a, t, g, st);
 }
+#endif
+
+#if DG_PART == 3
 
 // Elements from which the two passes beat the fused stage, whose single
 // launch is the shorter one while launches and latency count (us of a middle
@@ -3374,18 +3399,7 @@ hipError_t launch_stage_two_pass(int P, int flux, const StageArgs& a, void* scra
     return hipSuccess;
 }
 
-hipError_t launch_stage_corrected(int P, int flux, const StageArgs& a, const float* C, const KTables* t,
-                                  const KGeom& g, hipStream_t st) {
-    if (P != 1 || g.dim != 3 || g.mapped || g.fp32 || a.mode == MODE_RESIDUAL) return hipErrorInvalidValue;
-    dim3 grid(g.E), block(stage_team<1>());
-    switch (flux) {
-    case 0: hipLaunchKernelGGL((stage_corr_kernel<1, 0>), grid, block, 0, st, a, t, g, C); break;
-    case 1: hipLaunchKernelGGL((stage_corr_kernel<1, 1>), grid, block, 0, st, a, t, g, C); break;
-    default: hipLaunchKernelGGL((stage_corr_kernel<1, 2>), grid, block, 0, st, a, t, g, C); break;
-    }
-    return hipGetLastError();
-}
-
+#elif DG_PART == 2
 hipError_t launch_stage_batch(int P, int flux, int fp32, int proj, int variant, const BatchCase* cases,
                               const unsigned* blk_case, unsigned nblocks, int stage, const KTables* t, hipStream_t st) {
     if (nblocks == 0) return hipSuccess;
@@ -3393,6 +3407,7 @@ hipError_t launch_stage_batch(int P, int flux, int fp32, int proj, int variant, 
     return hipSuccess;
 }
 
+#elif DG_PART == 0
 int batch_team(int P, int variant) {
     switch (P) {
     case 1: return team_of<1>(variant);
@@ -3478,5 +3493,6 @@ hipError_t launch_mass(int P, double* imm, double* jmin, const KTables* t, const
     }
     return hipGetLastError();
 }
+#endif
 
 }  // namespace dg
