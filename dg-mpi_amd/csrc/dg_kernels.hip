@@ -3331,18 +3331,16 @@ hipError_t launch_stage(int P, int flux, const StageArgs& a, const KTables* t, c
 #if DG_PART == 3
 
 // Elements from which the two passes beat the fused stage, whose single
-// launch is the shorter one while launches and latency count (us of a middle
-// stage, two passes / fused, at the sizes on either side: FP64 p = 1 4096
-// 12.1 / 11.8, 8000 15.5 / 20.7; p = 2 1728 16.4 / 12.3, 4096 19.4 / 23.3;
-// p = 3 1728 24.7 / 20.3, 4096 34.6 / 38.4; FP32 p = 1 4096 12.4 / 10.2, 8000
-// 15.0 / 15.7; p = 2 4096 18.3 / 17.6, 8000 24.2 / 29.6; p = 4 19600 185 /
-// 183, 32768 281 / 384; p = 5 4096 81 / 79, 8000 145 / 151; the residual in FP64
-// p = 1 4624 11.8 / 14.0, p = 2 2730 16.4 / 17.9, p = 5 2940 68.7 / 82.0).
-// The FP32 form at p = 3 stays fused: there stage_kernel solves in the box's
-// frame, and the two passes' FP32 rounding would differ from it (at the other
-// orders the two agree to the bit).
+// launch is the shorter one while launches and latency count (us, two passes /
+// fused, at the sizes on either side; a middle stage: FP64 p = 1 4096 12.1 /
+// 11.8, 8000 15.5 / 20.7; p = 2 1728 16.4 / 12.3, 4096 19.4 / 23.3; p = 3 1728
+// 24.7 / 20.3, 4096 34.6 / 38.4; FP32 p = 1 4096 12.4 / 10.2, 8000 15.0 / 15.7;
+// p = 2 4096 18.3 / 17.6, 8000 24.2 / 29.6; p = 4 19600 185 / 183, 32768 281 /
+// 384; p = 5 4096 81 / 79, 8000 145 / 151; the residual: FP64 p = 1 4624 11.8 /
+// 14.0, p = 2 2730 16.4 / 17.9, p = 5 2940 68.7 / 82.0; FP32 p = 3 4096 29.2 /
+// 27.3, 5832 33.1 / 36.7)
 unsigned two_pass_min_elements(int P, int fp32) {
-    static const unsigned lim[2][PMAX] = {{4608, 2560, 2816, 2816, 2816}, {7168, 5120, ~0u, 24576, 6656}};
+    static const unsigned lim[2][PMAX] = {{4608, 2560, 2816, 2816, 2816}, {7168, 5120, 5120, 24576, 6656}};
     return P >= 1 && P <= PMAX ? lim[fp32 ? 1 : 0][P - 1] : ~0u;
 }
 
@@ -3369,15 +3367,7 @@ hipError_t launch_stage_two_pass_batch(int P, int flux, int fp32, BatchCase* cas
                                        unsigned face_blocks, const unsigned* elem_case, unsigned elem_blocks, int stage,
                                        const KTables* t, hipStream_t st) {
 #define DG_TWO(PP, R) two_pass_batch_p<PP, R>(flux, cases, face_case, face_blocks, elem_case, elem_blocks, stage, t, st)
-    if (fp32) {
-        switch (P) {
-        case 1: return DG_TWO(1, float);
-        case 2: return DG_TWO(2, float);
-        case 4: return DG_TWO(4, float);
-        case 5: return DG_TWO(5, float);
-        default: return hipErrorInvalidValue;
-        }
-    }
+    if (fp32) DG_DISPATCH_P(P, return DG_TWO(PP, float));
     DG_DISPATCH_P(P, return DG_TWO(PP, double));
 #undef DG_TWO
     return hipErrorInvalidValue;
@@ -3386,15 +3376,7 @@ hipError_t launch_stage_two_pass_batch(int P, int flux, int fp32, BatchCase* cas
 hipError_t launch_stage_two_pass(int P, int flux, const StageArgs& a, void* scratch, const float* corr,
                                  const KTables* t, const KGeom& g, hipStream_t st) {
     if (!scratch || g.dim != 3 || g.mapped || g.proj) return hipErrorInvalidValue;
-    if (g.fp32) {
-        switch (P) {
-        case 1: return two_pass_p<1, float>(flux, a, scratch, corr, t, g, st);
-        case 2: return two_pass_p<2, float>(flux, a, scratch, corr, t, g, st);
-        case 4: return two_pass_p<4, float>(flux, a, scratch, corr, t, g, st);
-        case 5: return two_pass_p<5, float>(flux, a, scratch, corr, t, g, st);
-        default: return hipErrorInvalidValue;
-        }
-    }
+    if (g.fp32) DG_DISPATCH_P(P, return (two_pass_p<PP, float>(flux, a, scratch, corr, t, g, st)));
     DG_DISPATCH_P(P, return (two_pass_p<PP, double>(flux, a, scratch, corr, t, g, st)));
     return hipSuccess;
 }

@@ -14,7 +14,7 @@ from dg_amd import hip
 pytestmark = pytest.mark.gpu
 
 # order, elements: in FP64 p = 1 takes over at 4608 elements, p = 2 at 2560,
-# the rest at 2816, in the FP32 form p = 1, 2, 4, 5 at 7168, 5120, 24576, 6656;
+# the rest at 2816, in the FP32 form at 7168, 5120, 5120, 24576, 6656;
 # the workgroups of the two passes hold 7 and 6, 5 and 4, 4 and 5, 3 and 3,
 # 3 and 2 elements
 CASES = [
@@ -23,6 +23,7 @@ CASES = [
     (2, (1, 2561, 1), "LegendreHex", "HLLC"),
     (3, (17, 13, 13), "LegendreHex", "Roe"), (3, (2819, 1, 1), "LagrangeHex", "HLLC"),
     (3, (14, 14, 14), "LegendreHex", "LaxFriedrichs"), (3, (18, 18, 18), "LagrangeHex", "Roe"),
+    (3, (19, 17, 17), "LegendreHex", "HLLC"), (3, (1, 32, 161), "LegendreHex", "LaxFriedrichs"),
     (4, (15, 14, 14), "LegendreHex", "HLLC"), (4, (23, 22, 23), "LagrangeHex", "Roe"),
     (4, (30, 29, 29), "LegendreHex", "LaxFriedrichs"),
     (5, (15, 15, 13), "LegendreHex", "Roe"), (5, (19, 19, 19), "LagrangeHex", "LaxFriedrichs"),
