@@ -172,8 +172,8 @@ __global__ void target_kernel(const double* __restrict__ Df, const double* __res
 // for the three layers, with the normalisation, GELU, de-normalisation and
 // the fallback bound around them.  The grid is persistent (at most one
 // block per CU): a block stages the three weight matrices once, transposed
-// to [output][input] in LDS, then walks 64-row tiles; wave w owns rows
-// 16w .. 16w+15 of a tile through all three layers.  Activations enter each
+// to [output][input] in LDS, then walks tiles of 16 rows per wave; a wave
+// takes its rows through all three layers by itself.  Activations enter each
 // layer rounded to bf16.
 //
 // Operand layout of the 16x16x16 bf16 MFMA (lane l, element q = 0..3):
@@ -181,21 +181,21 @@ __global__ void target_kernel(const double* __restrict__ Df, const double* __res
 // holds D[4 (l / 16) + q][l % 16].
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr int MT = 256, MR = 64;               // threads, rows per tile
 constexpr int K1 = 80;                         // layer-1 inputs padded to whole 16-wide k steps
 constexpr int L1S = K1 + 4, L2S = NH + 4;      // LDS row strides (bf16), padded off the bank period
 constexpr int N3 = 48;                         // layer-3 outputs padded to whole 16-column tiles
-constexpr int MAX_INFER_BLOCKS = 256;
+constexpr int WV = 64;                         // lanes per wave
+constexpr int MAX_INFER_BLOCKS = 256;          // a block per CU
 constexpr int GCHUNKS = 32;                   // most row chunks of one weight-gradient pass
 
+// WN pairs of waves with 16 rows each; the rows hold the features, then each
+// layer's activations and the de-normalised outputs in place
+template <int WN>
 struct InferLDS {
     uint16_t w1[NH][L1S];                      // W1^T; inputs k >= NF are zero
     uint16_t w2[NH][L2S];                      // W2^T
     uint16_t w3[N3][L2S];                      // W3^T; outputs n >= NO are zero
-    uint16_t a0[MR][L1S];                      // normalised features
-    uint16_t h1[MR][L2S];
-    uint16_t h2[MR][L2S];
-    float o[MR][NO + 1];                       // de-normalised outputs
+    uint16_t a[16 * WN][L2S];
 };
 
 __device__ inline bf16x4 ld_bf16x4(const uint16_t* q) { return *reinterpret_cast<const bf16x4*>(q); }
@@ -223,13 +223,13 @@ __global__ void pack_infer_weights(const uint16_t* __restrict__ W, uint16_t* __r
 }
 
 // acc[j] += A[16 rows][K] x W^T[16 j .. 16 j + 15][K] for j < NT
+// W^T from the rows of the first tile on
 template <int NT, int K, int LA, int LW>
-__device__ __forceinline__ void mfma_layer(const uint16_t (*A)[LA], const uint16_t (*Wt)[LW], int rw, int lane,
-                                           f32x4* acc) {
+__device__ __forceinline__ void mfma_layer(const uint16_t (*A)[LA], const uint16_t (*Wt)[LW], int lane, f32x4* acc) {
     const int c = lane & 15, kq = 4 * (lane >> 4);
-#pragma unroll
+#pragma unroll 2
     for (int kk = 0; kk < K; kk += 16) {
-        const bf16x4 a = ld_bf16x4(&A[rw + c][kk + kq]);
+        const bf16x4 a = ld_bf16x4(&A[c][kk + kq]);
 #pragma unroll
         for (int j = 0; j < NT; ++j)
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, ld_bf16x4(&Wt[16 * j + c][kk + kq]), acc[j], 0, 0,
@@ -237,18 +237,79 @@ __device__ __forceinline__ void mfma_layer(const uint16_t (*A)[LA], const uint16
     }
 }
 
-__global__ __launch_bounds__(MT) void mlp_infer_kernel(const float* __restrict__ X,
-                                                       const uint16_t* __restrict__ Wimg,
-                                                       const float* __restrict__ P, const float* __restrict__ xs,
-                                                       float* __restrict__ C, double bound, long rows,
-                                                       unsigned long long* __restrict__ count) {
-    __shared__ alignas(16) InferLDS L;
-    const int t = threadIdx.x, lane = t & 63, rw = 16 * (t >> 6);
-    const int c = lane & 15, rq = 4 * (lane >> 4);
+// Features of the elements r0 .. r0 + nr - 1 of a box, normalised and rounded,
+// into the 16 rows of a pair of waves (lane 0 .. 127; features_kernel's values: the 40 coefficients,
+// then per face the jump of the face mean).  A lane takes one variable and
+// direction of an element, both faces.
+__device__ __forceinline__ void pair_features(const double* __restrict__ U, const dg::KTables& T, const dg::KGeom& G,
+                                              const float* __restrict__ xs, long r0, int nr, int lane,
+                                              uint16_t (*a)[L2S]) {
+    auto put = [&](int r, int k, float x) { a[r][k] = to_bf16((x - xs[k]) * xs[NF + k]); };
+#pragma unroll
+    for (int t0 = 0; t0 < 16 * 40; t0 += 2 * WV) {
+        const int t = t0 + lane, r = t / 40;
+        if (r < nr) put(r, t - 40 * r, (float)U[r0 * 40 + t]);
+    }
+    double m[2], P[2][8];                      // weights of the - and + face means, b = r + 2 t1 + 4 t2
+    for (int jj = 0; jj < 2; ++jj) {
+        double v = 0.;
+        for (int g = 0; g < 3; ++g) v += T.w[g] * T.B[g][jj];
+        m[jj] = 0.5 * v;
+    }
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        P[0][b] = T.phim[b & 1] * m[b >> 1 & 1] * m[b >> 2];
+        P[1][b] = T.phip[b & 1] * m[b >> 1 & 1] * m[b >> 2];
+    }
+#pragma unroll 1
+    for (int t = lane; t < 16 * 15; t += 2 * WV) {
+        const int r = t / 15, ds = t - 15 * r, d = ds / 5, s = ds - 5 * d;
+        if (r >= nr) continue;
+        const unsigned e = (unsigned)(r0 + r), nx = G.ne[0], ny = G.ne[1], nz = G.ne[2];
+        const unsigned yz = e / nx, z = yz / ny;
+        const unsigned c = d == 0 ? e - yz * nx : (d == 1 ? yz - z * ny : z);
+        const unsigned st = d == 0 ? 1u : (d == 1 ? nx : nx * ny), n = d == 0 ? nx : (d == 1 ? ny : nz);
+        const unsigned em = e - st + (c == 0 ? st * n : 0u), ep = e + st - (c + 1 == n ? st * n : 0u);
+        const double *u = U + (size_t)e * 40 + s, *um = U + (size_t)em * 40 + s, *up = U + (size_t)ep * 40 + s;
+        double om = 0., op = 0., nm = 0., np = 0.;
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {          // mode b = i + 2 j + 4 k; its (r, t1, t2) along d
+            const int b1 = (b >> 1 & 1) | (b & 1) << 1 | (b & 4), b2 = (b >> 2) | (b & 1) << 1 | (b >> 1 & 1) << 2;
+            const double wm = d == 0 ? P[0][b] : (d == 1 ? P[0][b1] : P[0][b2]);
+            const double wp = d == 0 ? P[1][b] : (d == 1 ? P[1][b1] : P[1][b2]);
+            om = fma(u[b * 5], wm, om);
+            op = fma(u[b * 5], wp, op);
+            nm = fma(um[b * 5], wp, nm);
+            np = fma(up[b * 5], wm, np);
+        }
+        put(r, 40 + 10 * d + s, (float)(nm - om));
+        put(r, 45 + 10 * d + s, (float)(np - op));
+    }
+    for (int t = lane; t < 16 * (K1 - NF); t += 2 * WV) a[t / (K1 - NF)][NF + t % (K1 - NF)] = 0;
+}
+
+// Rows X (STATE: the features of the box state U) through the network; the two
+// waves of a pair take half of each layer's columns.  Bound: VALU issue, more
+// than half of it in the error functions (256 per row; 32 of some 50
+// instructions per lane).  32768 elements: 26.9 us with the features, against
+// 19.4 for a features kernel and 30.2 for four waves a block that took two
+// tiles one after the other.
+template <int WN, bool STATE>
+__global__ __launch_bounds__(2 * WN * WV) void mlp_infer_kernel(const float* __restrict__ X, const double* __restrict__ U,
+                                                                const dg::KTables* __restrict__ Tp, dg::KGeom G,
+                                                                const uint16_t* __restrict__ Wimg,
+                                                                const float* __restrict__ P,
+                                                                const float* __restrict__ xs, float* __restrict__ C,
+                                                                double bound, long rows,
+                                                                unsigned long long* __restrict__ count) {
+    constexpr int MT = 2 * WN * WV, MR = WN * 16;
+    __shared__ alignas(16) InferLDS<WN> L;
+    int t = threadIdx.x;
     // the weights' LDS image, a straight 16-byte copy
-    static_assert(offsetof(InferLDS, w2) == IMG1 * 2 && offsetof(InferLDS, w3) == (IMG1 + IMG2) * 2 &&
-                      IMG * 2 % 16 == 0,
+    static_assert(offsetof(InferLDS<WN>, w2) == IMG1 * 2 && offsetof(InferLDS<WN>, w3) == (IMG1 + IMG2) * 2 &&
+                      offsetof(InferLDS<WN>, a) == IMG * 2 && IMG * 2 % 16 == 0,
                   "contiguous weight image");
+    static_assert((NO + 1) * 4 <= L2S * 2 && K1 <= L2S, "outputs and features fit a row");
     {
         constexpr int NV = IMG * 2 / 16;
         const uint4* src = reinterpret_cast<const uint4*>(Wimg);
@@ -266,79 +327,89 @@ __global__ __launch_bounds__(MT) void mlp_infer_kernel(const float* __restrict__
     }
     const long ntile = (rows + MR - 1) / MR;
     for (long tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
-        const long r0 = tile * MR;
-        const int nr = (int)(rows - r0 < MR ? rows - r0 : MR);
-        __syncthreads();                       // the staged weights; the previous tile's a0 and o are read
-        {
-            // the tile's features: all global loads first, then the stores
-            constexpr int PER = (MR * K1 + MT - 1) / MT;
+        // nothing of a tile is kept over the loop (addresses and biases held
+        // in registers for the next tile, which is rare, spill)
+        asm volatile("" : "+v"(t));
+        asm volatile("" : "+s"(P), "+s"(xs));
+        const int lane = t & 63, pl = t & 127, half = t >> 6 & 1, pair = t >> 7;
+        const int c = lane & 15, rq = 4 * (lane >> 4);
+        uint16_t(*const a)[L2S] = L.a + 16 * pair;
+        const long r0 = tile * MR + 16 * pair;
+        const int nr = (int)(rows - r0 < 16 ? rows - r0 : 16);     // may be 0 or less in the last tile
+        if constexpr (!STATE) {
+            // the features: all global loads first, then the stores
+            constexpr int PER = 16 * K1 / (2 * WV);
             float xv[PER];
 #pragma unroll
             for (int u = 0; u < PER; ++u) {
-                const int i = t + u * MT, r = i / K1, k = i % K1;
-                xv[u] = (i < MR * K1 && r < nr && k < NF) ? X[(r0 + r) * NF + k] : 0.f;
+                const int i = pl + u * 2 * WV, r = i / K1, k = i % K1;
+                xv[u] = (r < nr && k < NF) ? X[(r0 + r) * NF + k] : 0.f;
             }
 #pragma unroll
             for (int u = 0; u < PER; ++u) {
-                const int i = t + u * MT, r = i / K1, k = i % K1;
-                if (i < MR * K1) L.a0[r][k] = (r < nr && k < NF) ? to_bf16((xv[u] - xs[k]) * xs[NF + k]) : (uint16_t)0;
+                const int i = pl + u * 2 * WV, r = i / K1, k = i % K1;
+                a[r][k] = (r < nr && k < NF) ? to_bf16((xv[u] - xs[k]) * xs[NF + k]) : (uint16_t)0;
             }
+        } else {
+            pair_features(U, *Tp, G, xs, r0, nr, pl, a);
         }
-        __syncthreads();
-        f32x4 acc[8];
-        // layer 1: NF -> NH, GELU
+        __syncthreads();                       // also the staged weights
+        // two hidden layers, GELU
+        f32x4 acc[4];
+        auto hidden = [&](auto first) {
+            constexpr bool one = decltype(first)::value;
+            const float* b = P + (one ? OFF_B1 : OFF_B2) + 64 * half;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float b = P[OFF_B1 + 16 * j + c];
-            acc[j] = f32x4{b, b, b, b};
-        }
-        mfma_layer<8, K1, L1S, L1S>(L.a0, L.w1, rw, lane, acc);
+            for (int j = 0; j < 4; ++j) acc[j] = f32x4{b[16 * j + c], b[16 * j + c], b[16 * j + c], b[16 * j + c]};
+            if constexpr (one) mfma_layer<4, K1, L2S, L1S>(a, L.w1 + 64 * half, lane, acc);
+            else mfma_layer<4, NH, L2S, L2S>(a, L.w2 + 64 * half, lane, acc);
+            __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
+            for (int j = 0; j < 4; ++j) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) L.h1[rw + rq + q][16 * j + c] = to_bf16(gelu(acc[j][q]));
-        __syncthreads();
-        // layer 2: NH -> NH, GELU
+                for (int q = 0; q < 4; ++q) a[rq + q][64 * half + 16 * j + c] = to_bf16(gelu(acc[j][q]));
+                __builtin_amdgcn_sched_barrier(0);     // four error functions in flight, not sixteen
+            }
+            __syncthreads();
+        };
+        hidden(std::true_type());
+        hidden(std::false_type());
+        // layer 3: NH -> NO, de-normalised; tiles 0 and 1, and tile 2
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float b = P[OFF_B2 + 16 * j + c];
-            acc[j] = f32x4{b, b, b, b};
-        }
-        mfma_layer<8, NH, L2S, L2S>(L.h1, L.w2, rw, lane, acc);
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) L.h2[rw + rq + q][16 * j + c] = to_bf16(gelu(acc[j][q]));
-        __syncthreads();
-        // layer 3: NH -> NO, de-normalised
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int n = 16 * j + c;
+        for (int j = 0; j < 2; ++j) {
+            const int n = 32 * half + 16 * j + c;
             const float b = n < NO ? P[OFF_B3 + n] : 0.f;
             acc[j] = f32x4{b, b, b, b};
         }
-        mfma_layer<3, NH, L2S, L2S>(L.h2, L.w3, rw, lane, acc);
+        if (half) mfma_layer<1, NH, L2S, L2S>(a, L.w3 + 32, lane, acc);
+        else mfma_layer<2, NH, L2S, L2S>(a, L.w3, lane, acc);
+        __syncthreads();
+        float* const o = reinterpret_cast<float*>(&a[0][0]);
+        constexpr int OS = L2S / 2;            // a row in floats
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int n = 16 * j + c;
+        for (int j = 0; j < 2; ++j) {
+            const int n = 32 * half + 16 * j + c;
             if (n < NO) {
                 const float ys = xs[2 * NF + n];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) L.o[rw + rq + q][n] = acc[j][q] * ys;
+                for (int q = 0; q < 4; ++q) o[(rq + q) * OS + n] = acc[j][q] * ys;
             }
         }
         __syncthreads();
         // fallback bound per row (count null: no bound), then the store
-        if (count && t < MR) {
-            double n2 = 0.;
-            for (int i = 0; i < NO; ++i) n2 += (double)L.o[t][i] * L.o[t][i];
-            if (t < nr && !(sqrt(n2) <= bound)) {
-                for (int i = 0; i < NO; ++i) L.o[t][i] = 0.f;
-                atomicAdd(count, 1ull);
+        if (count) {
+            if (pl < nr) {
+                double n2 = 0.;
+                for (int i = 0; i < NO; ++i) n2 += (double)o[pl * OS + i] * o[pl * OS + i];
+                if (!(sqrt(n2) <= bound)) {
+                    for (int i = 0; i < NO; ++i) o[pl * OS + i] = 0.f;
+                    atomicAdd(count, 1ull);
+                }
             }
+            __syncthreads();
         }
-        __syncthreads();
-        for (int i = t; i < nr * NO; i += MT) C[r0 * NO + i] = L.o[i / NO][i % NO];
+        for (int i = pl; i < nr * NO; i += 2 * WV) C[r0 * NO + i] = o[i / NO * OS + i % NO];
+        __syncthreads();                       // the rows are free for the next tile
     }
 }
 
@@ -351,7 +422,6 @@ __global__ __launch_bounds__(MT) void mlp_infer_kernel(const float* __restrict__
 // arithmetic is that of a plain FP32 network with bf16 weights up to the
 // order of the FP32 sums.
 // ---------------------------------------------------------------------------
-constexpr int WV = 64;                         // lanes per wave
 constexpr int RT = 16;                         // rows of a train_rows workgroup
 constexpr int RW = NH / 16;                    // its waves: a 16-column tile of the hidden layers each
 constexpr int RB = RW * WV;
@@ -688,18 +758,17 @@ __global__ void target_at_kernel(const double* __restrict__ Df, const double* __
     Y[t] = (float)(Df[f] - Dc[t] + (Uf[f] - Uc[t]) * rtau);
 }
 
-// Device scratch of dg_closure_step_noalloc: the feature rows [E][NF], the
-// corrections [E][NO] and the 64-bit fallback counter of up to
-// NOALLOC_MAX_ELEMS elements (32^3, the closure's box), 14.4 MB, in a
+// Device scratch of dg_closure_step_noalloc: the corrections [E][NO] and the
+// 64-bit fallback counter of up to NOALLOC_MAX_ELEMS elements (32^3, the
+// closure's box), 5.2 MB, in a
 // file-scope array that each GPU holds until the process ends.  Host code
 // never passes the array's name to a kernel (on the host it is a stand-in,
 // not a device address): it uses the address hipGetSymbolAddress returns
 // for the current device (noalloc_scratch).
 constexpr long NOALLOC_MAX_ELEMS = 32768;
-constexpr size_t NOALLOC_X = (size_t)NOALLOC_MAX_ELEMS * NF;        // floats
 constexpr size_t NOALLOC_C = (size_t)NOALLOC_MAX_ELEMS * NO;        // floats
-constexpr size_t NOALLOC_FLOATS = NOALLOC_X + NOALLOC_C + 2;        // + the counter (8 B, 8-aligned)
-static_assert(((NOALLOC_X + NOALLOC_C) * sizeof(float)) % 8 == 0, "counter alignment");
+constexpr size_t NOALLOC_FLOATS = NOALLOC_C + 2;        // + the counter (8 B, 8-aligned)
+static_assert((NOALLOC_C * sizeof(float)) % 8 == 0, "counter alignment");
 static __device__ __align__(256) float scratch[NOALLOC_FLOATS];
 
 // one thread clears *p (a vector store: the address is lane-indexed)
@@ -748,19 +817,32 @@ void free_acts(dg_mlp* m) {
     m->cap = 0;
 }
 
-// the inference kernel on a persistent grid of at most one block per CU
-// (the weight image is rebuilt first, on the same stream, when pb changed)
-void launch_infer(dg_mlp* m, const float* X, float* C, double bound, long rows, unsigned long long* count,
-                  hipStream_t st) {
+// The inference kernel on a persistent grid of at most one block per CU (the
+// weight image is rebuilt first, on the same stream, when pb changed), on rows
+// X, or for null X on the features of the state U of the box s.  Four pairs
+// of waves a block while that is a tile per CU; above, eight share the staged
+// weights (one tile per CU in place of two one after the other).
+void launch_infer(dg_mlp* m, const float* X, const dg_solver* s, const double* U, float* C, double bound, long rows,
+                  unsigned long long* count, hipStream_t st) {
     if (m->img_stale) {
         hipLaunchKernelGGL(pack_infer_weights, dim3(nblk(IMG)), dim3(TB), 0, st, m->pb, m->img);
         hcheck(hipGetLastError(), "weight image kernel");
         m->img_stale = false;
     }
-    const long ntile = (rows + MR - 1) / MR;
-    const unsigned grid = (unsigned)(ntile < MAX_INFER_BLOCKS ? ntile : MAX_INFER_BLOCKS);
-    hipLaunchKernelGGL(mlp_infer_kernel, dim3(grid), dim3(MT), 0, st, X, m->img, m->p, m->xs, C, bound, rows,
-                       count);
+    const dg::KTables* tab = s ? s->dtab : nullptr;
+    const dg::KGeom g = s ? s->geo : dg::KGeom{};
+    auto launch = [&](auto waves, auto state) {
+        constexpr int WN = decltype(waves)::value;
+        const long ntile = (rows + 16 * WN - 1) / (16 * WN);
+        const unsigned grid = (unsigned)(ntile < MAX_INFER_BLOCKS ? ntile : MAX_INFER_BLOCKS);
+        hipLaunchKernelGGL((mlp_infer_kernel<WN, decltype(state)::value>), dim3(grid), dim3(2 * WN * WV), 0, st, X, U, tab, g, m->img, m->p, m->xs, C,
+                           bound, rows, count);
+    };
+    const bool few = rows <= 4 * 16 * MAX_INFER_BLOCKS;
+    std::integral_constant<int, 4> w4;
+    std::integral_constant<int, 8> w8;
+    if (X) few ? launch(w4, std::false_type()) : launch(w8, std::false_type());
+    else few ? launch(w4, std::true_type()) : launch(w8, std::true_type());
     hcheck(hipGetLastError(), "inference kernel");
 }
 
@@ -923,9 +1005,9 @@ double closure_check(dg_solver* s, dg_mlp* m, double dt_step, int nsteps) {
     return dt;
 }
 
-// nsteps corrected RK4 steps with the given feature rows X [E][NF],
-// corrections C [E][NO] and fallback counter cnt (device memory)
-void closure_steps(dg_solver* s, dg_mlp* m, double dt, double bound, int nsteps, float* X, float* C,
+// nsteps corrected RK4 steps with the given corrections C [E][NO] and fallback
+// counter cnt (device memory)
+void closure_steps(dg_solver* s, dg_mlp* m, double dt, double bound, int nsteps, float* C,
                    unsigned long long* cnt, long* n_fallback) {
     const long E = s->geo.E;
     // the counter is cleared by a kernel (no memset node if the caller
@@ -935,11 +1017,10 @@ void closure_steps(dg_solver* s, dg_mlp* m, double dt, double bound, int nsteps,
     // the network's parameters are written by its own stream (training)
     hcheck(hipStreamSynchronize(m->stream), "hipStreamSynchronize");
     auto stage = [&](const double* Ust, double* Uout, int mode, double alpha) {
-        // everything on the solver's stream: features, the network with
-        // its fallback, and the stage kernel whose RK epilogue takes
+        // everything on the solver's stream: the network on the state's
+        // features with its fallback, and the stage kernel whose RK epilogue takes
         // dU = dt (M^-1 R + C)
-        hipLaunchKernelGGL(features_kernel, dim3(nblk(E * FT)), dim3(TB), 0, s->stream, Ust, X, s->dtab, s->geo);
-        launch_infer(m, X, C, bound, E, cnt, s->stream);
+        launch_infer(m, nullptr, s, Ust, C, bound, E, cnt, s->stream);
         dg::StageArgs a{};
         a.Ust = Ust;
         a.U0 = s->U0;
@@ -1089,7 +1170,7 @@ int dg_mlp_forward(dg_mlp* m, const float* X_dev, float* Y_dev, long rows) {
         if (rows < 1) throw std::invalid_argument("rows < 1");
         hcheck(hipSetDevice(m->device), "hipSetDevice");
         // the closure step's inference kernel, without the fallback bound
-        launch_infer(m, X_dev, Y_dev, 0.0, rows, nullptr, m->stream);
+        launch_infer(m, X_dev, nullptr, nullptr, Y_dev, 0.0, rows, nullptr, m->stream);
         hcheck(hipStreamSynchronize(m->stream), "hipStreamSynchronize");
     });
 }
@@ -1213,12 +1294,11 @@ int dg_closure_step(dg_solver* s, dg_mlp* m, double dt_step, double bound, int n
     return mlp_guard(g_mlp_error, [&] {
         const double dt = closure_check(s, m, dt_step, nsteps);
         const long E = s->geo.E;
-        // the feature rows, corrections and counter live on the solver
-        // handle from the first call on (freed by dg_destroy)
-        if (!s->cl_X) hcheck(hipMalloc(&s->cl_X, (size_t)E * NF * sizeof(float)), "hipMalloc");
+        // the corrections and the counter live on the solver handle from the
+        // first call on (freed by dg_destroy)
         if (!s->cl_C) hcheck(hipMalloc(&s->cl_C, (size_t)E * NO * sizeof(float)), "hipMalloc");
         if (!s->cl_cnt) hcheck(hipMalloc(&s->cl_cnt, sizeof(unsigned long long)), "hipMalloc");
-        closure_steps(s, m, dt, bound, nsteps, s->cl_X, s->cl_C, s->cl_cnt, n_fallback);
+        closure_steps(s, m, dt, bound, nsteps, s->cl_C, s->cl_cnt, n_fallback);
     });
 }
 
@@ -1231,10 +1311,9 @@ int dg_closure_step_noalloc(dg_solver* s, dg_mlp* m, double dt_step, double boun
                                         std::to_string(NOALLOC_MAX_ELEMS) + " of its static scratch (use dg_closure_step)");
         // the device is current (closure_check): its own copy of the array
         float* base = noalloc_scratch(s->device);
-        float* X = base;
-        float* C = base + NOALLOC_X;
-        auto* cnt = reinterpret_cast<unsigned long long*>(base + NOALLOC_X + NOALLOC_C);
-        closure_steps(s, m, dt, bound, nsteps, X, C, cnt, n_fallback);
+        float* C = base;
+        auto* cnt = reinterpret_cast<unsigned long long*>(base + NOALLOC_C);
+        closure_steps(s, m, dt, bound, nsteps, C, cnt, n_fallback);
     });
 }
 

@@ -200,10 +200,9 @@ void free_all(dg_solver* s) {
     s->nev = nullptr;
     if (s->dtab) (void)hipFree(s->dtab);
     s->dtab = nullptr;
-    if (s->cl_X) (void)hipFree(s->cl_X);
     if (s->cl_C) (void)hipFree(s->cl_C);
     if (s->cl_cnt) (void)hipFree(s->cl_cnt);
-    s->cl_X = s->cl_C = nullptr;
+    s->cl_C = nullptr;
     s->cl_cnt = nullptr;
     if (s->own_stream) (void)hipStreamDestroy(s->own_stream);
     s->U0 = s->Ua = s->Ub = s->acc = s->work = s->X = s->imm = nullptr;

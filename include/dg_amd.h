@@ -288,8 +288,8 @@ int dg_closure_step(dg_solver* s, dg_mlp* m, double dt, double bound, int nsteps
 /* dg_closure_step without any memory allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc).  The feature rows, corrections and fallback counter live in
- * a static device array of the library (14.4 MB, held by each GPU the
+ * hipMalloc).  The corrections and the fallback counter live in
+ * a static device array of the library (5.2 MB, held by each GPU the
  * library runs on until the process ends) instead of buffers on the
  * handle; it takes at most 32768 elements (32^3) and returns
  * DG_ERR_ARGUMENT above that.  Every call on one GPU shares that GPU's
