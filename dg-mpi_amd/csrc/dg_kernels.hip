@@ -1270,10 +1270,10 @@ __device__ __forceinline__ void face_phase(const KTables& T, const LaneTabT<R>& 
 // ---------------------------------------------------------------------------
 // Volume phase: sum-factorised interpolation, point fluxes, weak gradient.
 // ---------------------------------------------------------------------------
-template <int P, int TS, bool MAPPED = false, class R = double>
+template <int P, int TS, bool MAPPED, class R, class MID>
 __device__ __forceinline__ void volume_phase(const KTables& T, const LaneTabT<R>& LT, const KGeom& G, int lane,
                                              R* sR, R* bankA, R* bankB,
-                                             const double* XL = nullptr) {
+                                             const double* XL, MID&& mid) {
     using Dm = Dims<P>;
     constexpr int N = Dm::N, M = Dm::M, NN = Dm::NN, MM = Dm::MM, MMM = Dm::MMM;
     const R* sU = bankA;
@@ -1426,6 +1426,7 @@ __device__ __forceinline__ void volume_phase(const KTables& T, const LaneTabT<R>
             Cc[((2 * N + k) * MM + ba) * V + s] = zz[k];
         }
     });
+    mid();
     sync();
     // b-step: along y (B for x and z fluxes, D for the y flux)
     team_for<N * M * V, TS>(lane, [&](int t) {
@@ -2428,42 +2429,89 @@ struct BoxNbr {
 // 124-139): r <- imm r with the element's symmetric inverse mass matrix in
 // global memory (row b' contiguous, imm[b'][b] = imm[b][b'], so threads of
 // consecutive b read consecutive addresses).  The sum over b' is split in
-// up to four chunks over the threads; part holds chunks * NB * V doubles.
+// up to four chunks over the threads; part holds PART doubles.  The 32 KB per
+// element at p = 3 are most of a stage's bytes, so a lane fetches 16 entries
+// at a time and the stage the first of them before the residual is there.
+// (24 x 20 x 22 warped elements at p = 3, RK4 step: 927 us with the entries
+// loaded where they are used, four round trips one after the other, 651 us.)
 template <int P, int TS>
-constexpr int dense_part_size() {
-    constexpr int NB = Dims<P>::NNN;
-    constexpr int CH0 = TS / NB;
-    constexpr int CH = CH0 < 1 ? 1 : (CH0 > 4 ? 4 : CH0);
-    return CH * NB * V;
-}
+struct DenseMinv {
+    static constexpr int NB = Dims<P>::NNN;
+    static constexpr int CH0 = TS / NB, CH = CH0 < 1 ? 1 : (CH0 > 4 ? 4 : CH0);
+    static constexpr int LEN = (NB + CH - 1) / CH;
+    static constexpr int PART = CH * NB * V;
+    static constexpr int TASKS = NB * CH, ROUNDS = (TASKS + TS - 1) / TS;
+    // entries of a lane's column in flight together, and those of its first
+    // task that load() fetches ahead of the residual
+    static constexpr int AHEAD = LEN < 16 ? LEN : 16;
+    double m[AHEAD];
+
+    static __device__ __forceinline__ void task(int t, int& b, int& b0, int& len) {
+        const int tc = TASKS % TS == 0 || t < TASKS ? t : TASKS - 1, ch = tc / NB;
+        b = tc % NB;
+        b0 = ch * LEN;
+        len = CH * LEN == NB || NB - b0 > LEN ? LEN : NB - b0;
+    }
+    // entries i0 .. of the column (past its end: the last one again)
+    static __device__ __forceinline__ void fetch(const double* __restrict__ col, int i0, int len, double* v) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            const bool in = (CH * LEN == NB && i0 + AHEAD <= LEN) || i0 + i < len;
+            v[i] = col[(size_t)(in ? i0 + i : len - 1) * NB];
+        }
+    }
+    __device__ __forceinline__ void load(const double* __restrict__ imm, int lane) {
+        int b, b0, len;
+        task(lane, b, b0, len);
+        fetch(imm + (size_t)b0 * NB + b, 0, len, m);
+    }
+    __device__ __forceinline__ void apply(const double* __restrict__ imm, int lane, double* r, double* part) {
+#pragma unroll
+        for (int rd = 0; rd < ROUNDS; ++rd) {
+            const int t = rd * TS + lane;
+            int b, b0, len;
+            task(t, b, b0, len);
+            const double* col = imm + (size_t)b0 * NB + b;
+            if (rd > 0) fetch(col, 0, len, m);
+            double acc[V] = {0., 0., 0., 0., 0.};
+#pragma unroll 1
+            for (int i0 = 0; i0 < LEN; i0 += AHEAD) {
+                double nx[AHEAD];
+                if (i0 + AHEAD < LEN) fetch(col, i0 + AHEAD, len, nx);
+#pragma unroll
+                for (int i = 0; i < AHEAD; ++i)
+                    if ((CH * LEN == NB && LEN % AHEAD == 0) || i0 + i < len) {
+                        const double* x = r + (b0 + i0 + i) * V;
+#pragma unroll
+                        for (int s = 0; s < V; ++s) acc[s] = fma(m[i], x[s], acc[s]);
+                    }
+                if (i0 + AHEAD < LEN) {
+#pragma unroll
+                    for (int i = 0; i < AHEAD; ++i) m[i] = nx[i];
+                }
+            }
+            if (TASKS % TS == 0 || t < TASKS) {
+#pragma unroll
+                for (int s = 0; s < V; ++s) part[t * V + s] = acc[s];
+            }
+        }
+        sync();
+        team_for<NB * V, TS>(lane, [&](int t) {
+            const int b = t / V, s = t % V;
+            double v = 0.;
+#pragma unroll
+            for (int ch = 0; ch < CH; ++ch) v += part[(ch * NB + b) * V + s];
+            r[t] = v;
+        });
+        sync();
+    }
+};
 
 template <int P, int TS>
 __device__ __forceinline__ void dense_minv(const double* __restrict__ imm, int lane, double* r, double* part) {
-    constexpr int NB = Dims<P>::NNN;
-    constexpr int CH0 = TS / NB;
-    constexpr int CH = CH0 < 1 ? 1 : (CH0 > 4 ? 4 : CH0);
-    constexpr int LEN = (NB + CH - 1) / CH;
-    team_for<NB * CH, TS>(lane, [&](int t) {
-        const int b = t % NB, ch = t / NB;
-        const int b0 = ch * LEN, b1 = b0 + LEN < NB ? b0 + LEN : NB;
-        double acc[V] = {0., 0., 0., 0., 0.};
-        for (int bp = b0; bp < b1; ++bp) {
-            const double m = imm[(size_t)bp * NB + b];
-#pragma unroll
-            for (int s = 0; s < V; ++s) acc[s] = fma(m, r[bp * V + s], acc[s]);
-        }
-#pragma unroll
-        for (int s = 0; s < V; ++s) part[(ch * NB + b) * V + s] = acc[s];
-    });
-    sync();
-    team_for<NB * V, TS>(lane, [&](int t) {
-        const int b = t / V, s = t % V;
-        double v = 0.;
-#pragma unroll
-        for (int ch = 0; ch < CH; ++ch) v += part[(ch * NB + b) * V + s];
-        r[t] = v;
-    });
-    sync();
+    DenseMinv<P, TS> M;
+    M.load(imm, lane);
+    M.apply(imm, lane, r, part);
 }
 
 // R = float: the FP32 form -- the face and volume phases (traces, fluxes,
@@ -2567,9 +2615,13 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const KTables& T,
     else if constexpr (WAVE_NBR) bn.store_slabs(LT, T.one_kind, bankB, lane);
     else pf.store_neighbour_slabs(LT, T.one_kind, bankB, lane);
     sync();
+    DenseMinv<MAPPED ? P : 1, TS> minv;
+    const double* const imm = MAPPED ? G.imm + (size_t)e * Dm::NNN * Dm::NNN : nullptr;
     if constexpr (MAPPED) {
         face_phase<P, FLUX, TS, MAPPED, R>(T, LT, G, lane, bankA, sR, bankA, bankB, XL, e);
-        volume_phase<P, TS, MAPPED, R>(T, LT, G, lane, sR, bankA, bankB, XL);
+        volume_phase<P, TS, MAPPED, R>(T, LT, G, lane, sR, bankA, bankB, XL, [&] {
+            if (rk) minv.load(imm, lane);
+        });
     } else {
         face_phase_box<P, FLUX, TS>(T, LT, G, rf, dc, lane, bankA, sR, bankA, bankB);
         volume_phase_box<P, TS, box_rounds<P, TS>(), R, PROJ>(T, G, rf, dc, lane, sR, bankA, bankB);
@@ -2604,7 +2656,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const KTables& T,
     const size_t base = (size_t)e * NB;
     const int mode = MODE >= 0 ? MODE : A.mode;
     if constexpr (MAPPED) {
-        if (rk) dense_minv<P, TS>(G.imm + (size_t)e * Dm::NNN * Dm::NNN, lane, sR, bankA);
+        if (rk) minv.apply(imm, lane, sR, bankA);
     } else {
         if (rk && !T.minv_diag) minv_lines<P, TS>(T, lane, sRd);
     }
@@ -2720,7 +2772,7 @@ __global__ __launch_bounds__(WAVE) void inv_mass_kernel(double dt, const double*
     const KTables& T = *Tp;
     constexpr int NB = Dims<P>::NNN * V;
     __shared__ double sR[NB];
-    __shared__ double part[dense_part_size<P, WAVE>()];
+    __shared__ double part[DenseMinv<P, WAVE>::PART];
     const int lane = threadIdx.x;
     const size_t base = (size_t)blockIdx.x * NB;
     team_for<NB>(lane, [&](int t) { sR[t] = R[base + t]; });
@@ -2793,7 +2845,7 @@ __global__ __launch_bounds__(WAVE) void init_state_kernel(double time, double* U
     __shared__ double fs[Q * Q * V];
     __shared__ double t1[Q * N * V];
     __shared__ double Xe[24];
-    __shared__ double part[dense_part_size<P, WAVE>()];
+    __shared__ double part[DenseMinv<P, WAVE>::PART];
     const int lane = threadIdx.x;
     const unsigned e = blockIdx.x;
     int ec[3];
