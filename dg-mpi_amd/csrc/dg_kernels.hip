@@ -1870,7 +1870,7 @@ __device__ __forceinline__ void face_phase_box(const KTables& T, const LaneTabT<
     sync();
 }
 
-template <int P, int TS, int NR, class R, int PROJ = 0>
+template <int P, int TS, int NR, class R, int PROJ = 0, bool HALVES = false>
 __device__ __forceinline__ void volume_phase_box(const KTables& T, const KGeom& G, const SplitRef<R>& rf,
                                                  const TaskDec<TS, NR>& dc, int lane, R* sR, R* bankA,
                                                  R* bankB) {
@@ -2129,6 +2129,7 @@ __device__ __forceinline__ void volume_phase_box(const KTables& T, const KGeom& 
         }
     });
     sync();
+    if constexpr (HALVES) sync();   // the other half's last step starts the residual
     // a-step: along x (Dw for the x flux, Bw for the others), into sR
     team_qs<NN * V, TS>(dc, lane, [&](int q, int s, int) {
         R y1[M], y2[M];
@@ -2556,8 +2557,21 @@ __device__ __forceinline__ void dense_minv(const double* __restrict__ imm, int l
 // which read and write the FP64 registers.  Periodic box only.
 // CORR: the RK update takes dU = dt (M^-1 R + C), C a per-DOF correction in
 // FP32 laid out like the state (the learned closure's corrected stage)
+// LDS of the stage whose halves work side by side (HALVES): the volume term's
+// bank A over the element's block, the face term's banks, the volume term's
+// bank B.  The residual starts over the face term's bank B, which its last
+// step no longer reads.
+template <int P>
+struct HalvesLDS {
+    using L = BoxLDS<P, 0, double>;
+    static constexpr int VA = cmax(cmax(L::U, L::X2), cmax(L::QD, L::BV));
+    static constexpr int FA = cmax(cmax(L::F1, L::FH), L::L2), FB = cmax(cmax(L::SLAB, L::F2), L::L1);
+    static constexpr int VB = cmax(cmax(L::X1, L::UQ), L::C);
+    static_assert(FB >= L::R, "the residual fits the face term's bank");
+    static constexpr int TOTAL = VA + FA + FB + VB;
+};
 template <int P, int FLUX, bool MAPPED, class R, int TS = stage_team<P>(), bool CORR = false, int PROJ = 0,
-          int MODE = -1>
+          int MODE = -1, bool HALVES = false>
 __device__ __forceinline__ void stage_body(const StageArgs& A, const KTables& T, const KGeom& G, unsigned e,
                                            const int* ec, const float* __restrict__ Corr = nullptr) {
     static_assert(sizeof(R) == 8 || !MAPPED, "the FP32 form is for the periodic box");
@@ -2568,16 +2582,17 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const KTables& T,
     using PF = StageLoads<P, TS>;
     constexpr int NB = Dm::NNN * V;
     constexpr int LA = MAPPED ? L::A : LB::A;
-    constexpr int LTOT = MAPPED ? L::TOTAL : LB::TOTAL;
+    using LH = HalvesLDS<HALVES ? P : 1>;
+    constexpr int LTOT = HALVES ? LH::TOTAL : (MAPPED ? L::TOTAL : LB::TOTAL);
     static_assert(sizeof(R) == 8 || LA * sizeof(R) >= NB * sizeof(double), "FP64 residual fits bank A");
     __shared__ alignas(16) R lds[LTOT];
     __shared__ LaneTabT<R> LT;
     // general path: the trilinear maps' coefficients of the element and of its
     // six face neighbours (slot d*2 + side), for the left elements' normals
     __shared__ double XL[MAPPED ? 168 : 1];
-    R* sR = lds;
-    R* bankA = lds + L::R;
-    R* bankB = bankA + LA;
+    R* sR = HALVES ? lds + LH::VA + LH::FA : lds;
+    R* bankA = HALVES ? lds : lds + L::R;
+    R* bankB = HALVES ? sR : bankA + LA;
     const int lane = threadIdx.x;
     const bool rk = (MODE >= 0 ? MODE : A.mode) != MODE_RESIDUAL;
     const TaskDec<TS, box_rounds<P, TS>()> dc(lane);
@@ -2660,8 +2675,24 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const KTables& T,
             if (rk) minv.load(imm, lane);
         });
     } else {
-        face_phase_box<P, FLUX, TS>(T, LT, G, rf, dc, lane, bankA, sR, bankA, bankB);
-        volume_phase_box<P, TS, box_rounds<P, TS>(), R, PROJ>(T, G, rf, dc, lane, sR, bankA, bankB);
+        if constexpr (HALVES) {
+            // wave-uniform halves with the same number of barriers (8): the
+            // face steps, and the volume steps on the block and banks of
+            // their own
+            static_assert(PROJ == 0 && sizeof(R) == 8, "the FP64 stage");
+            constexpr int HT = TS / 2, HR = box_rounds<P, HT>();
+            const int hl = lane % HT;
+            const TaskDec<HT, HR> hc(hl);
+            if (__builtin_amdgcn_readfirstlane(lane / HT) == 0) {
+                face_phase_box<P, FLUX, HT>(T, LT, G, rf, hc, hl, bankA, sR, lds + LH::VA - BoxLDS<P>::U, bankB);
+                sync();
+            } else {
+                volume_phase_box<P, HT, HR, R, 0, true>(T, G, rf, hc, hl, sR, bankA, bankB + LH::FB);
+            }
+        } else {
+            face_phase_box<P, FLUX, TS>(T, LT, G, rf, dc, lane, bankA, sR, bankA, bankB);
+            volume_phase_box<P, TS, box_rounds<P, TS>(), R, PROJ>(T, G, rf, dc, lane, sR, bankA, bankB);
+        }
     }
     // FP32 form: the residual widened to FP64 in LDS (bank A is free again)
     // where M^-1 mixes coefficients; a diagonal M^-1 scales each lane's own
@@ -2750,6 +2781,20 @@ void stage_kernel(StageArgs A, const KTables* __restrict__ Tp,
     int ec[3];
     const unsigned e = block_element_xyz(G, ec);
     stage_body<P, FLUX, MAPPED, R, stage_team<P>(), false, PROJ, MODE>(A, *Tp, G, e, ec);
+}
+
+// The FP64 box stage for boxes of a few elements per CU, where a stage is one
+// workgroup's chain of steps (warm caches and a kernel shared by the stages
+// did not shorten it): half of the workgroup takes the face term, the other
+// half, HT threads too, the volume term, 8 steps between barriers instead of
+// 14, with the same sums.  A stage, 8^3 elements: p = 1 6.98 -> 6.00 us, p = 2
+// 8.79 -> 7.50, p = 3 10.6 -> 9.8.
+template <int P, int FLUX, int MODE, int HT>
+__global__ __launch_bounds__(2 * HT)
+void stage_halves_kernel(StageArgs A, const KTables* __restrict__ Tp, KGeom G) {
+    int ec[3];
+    const unsigned e = block_element_xyz(G, ec);
+    stage_body<P, FLUX, false, double, 2 * HT, false, 0, MODE, true>(A, *Tp, G, e, ec);
 }
 
 // The closure's corrected RK stage on an affine FP64 box (RK modes only)
@@ -3157,11 +3202,44 @@ __global__ __launch_bounds__(256) void mass_kernel(double* imm, double* jmin, co
 // ---------------------------------------------------------------------------
 // Dispatch
 // ---------------------------------------------------------------------------
+// Threads per half of stage_halves_kernel, or 0 for stage_kernel, whose
+// workgroups pack a filled chip better (us per stage, halves / whole: p = 1
+// 1728 elements 7.8 / 8.3, 2744 10.4 / 9.7; p = 2 1000 9.2 / 9.5, 1331 12.7 /
+// 12.5; p = 3, which three workgroups' LDS per CU limit, 729 11.7 / 12.2, 1000
+// 15.7 / 13.6, with halves of 256 threads 216 7.6 / 8.9, 512 9.8 / 10.6, 693
+// 14.0 / 12.5)
+template <int P>
+int halves_team(unsigned E) {
+    if (P == 1) return E <= 2048 ? 64 : 0;
+    if (P == 2) return E <= 1024 ? 128 : 0;
+    return E <= 512 ? 256 : (E <= 768 ? 128 : 0);
+}
+
+template <int P, int FLUX, int HT>
+void stage_halves_mode(const StageArgs& a, const KTables* t, const KGeom& g, dim3 grid, hipStream_t st) {
+    const dim3 block(2 * HT);
+    switch (a.mode) {
+    case MODE_RK_FIRST: hipLaunchKernelGGL((stage_halves_kernel<P, FLUX, MODE_RK_FIRST, HT>), grid, block, 0, st, a, t, g); break;
+    case MODE_RK_MID: hipLaunchKernelGGL((stage_halves_kernel<P, FLUX, MODE_RK_MID, HT>), grid, block, 0, st, a, t, g); break;
+    case MODE_RK_LAST: hipLaunchKernelGGL((stage_halves_kernel<P, FLUX, MODE_RK_LAST, HT>), grid, block, 0, st, a, t, g); break;
+    case MODE_FE: hipLaunchKernelGGL((stage_halves_kernel<P, FLUX, MODE_FE, HT>), grid, block, 0, st, a, t, g); break;
+    default: hipLaunchKernelGGL((stage_halves_kernel<P, FLUX, MODE_RESIDUAL, HT>), grid, block, 0, st, a, t, g); break;
+    }
+}
+
 // Box stage (FP64 or the FP32 form) with the RK mode compiled in (its
 // epilogue then has no mode selects); the residual mode keeps the run-time
 // form
 template <int P, int FLUX, class R>
 void stage_box_mode(const StageArgs& a, const KTables* t, const KGeom& g, dim3 grid, dim3 block, hipStream_t st) {
+    if constexpr (sizeof(R) == 8 && P <= 3) {
+        if (const int ht = halves_team<P>(g.E)) {
+            if constexpr (P == 1) stage_halves_mode<P, FLUX, 64>(a, t, g, grid, st);
+            else if (ht == 128) stage_halves_mode<P, FLUX, 128>(a, t, g, grid, st);
+            else if constexpr (P == 3) stage_halves_mode<P, FLUX, 256>(a, t, g, grid, st);
+            return;
+        }
+    }
     switch (a.mode) {
     case MODE_RK_FIRST: hipLaunchKernelGGL((stage_kernel<P, FLUX, false, R, 0, MODE_RK_FIRST>), grid, block, 0, st, a, t, g); break;
     case MODE_RK_MID: hipLaunchKernelGGL((stage_kernel<P, FLUX, false, R, 0, MODE_RK_MID>), grid, block, 0, st, a, t, g); break;
