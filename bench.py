@@ -661,9 +661,10 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": measured_traffic() if headline else None},
-        "kernel": {"name": f"stage_kernel<{order},Roe{',mapped' if args.warp else ''}{',fp32' if args.fp32 else ''}>"
+        "kernel": {"name": (f"stage_kernel<{order},Roe,mapped>" if args.warp else
+                            f"face_flux_kernel<{order},Roe>+element_kernel<{order}>{',fp32' if args.fp32 else ''}")
                    if dim == 3 else
-                   f"stage2d_kernel<{order},Roe>",
+                   f"stage2d_box_kernel<{order},Roe>",
                    "avg_launch_ms": ms_per_step / 4,
                    "launches": 4 * args.steps, "alg_bytes_per_launch": bytes_per_launch,
                    "alg_flops_per_launch": flops_launch,
