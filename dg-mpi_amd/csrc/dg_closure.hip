@@ -850,16 +850,16 @@ void ensure_acts(dg_mlp* m, long rows) {
     rows = (rows + RT - 1) / RT * RT;          // train_rows writes whole tiles
     if (rows <= m->cap) return;
     free_acts(m);
-    auto al = [&](float** q, long n) { hcheck(hipMalloc(q, (size_t)n * sizeof(float)), "hipMalloc(mlp)"); };
+    auto al = [&](float** q, long n) { hcheck(dg::device_malloc(q, (size_t)n * sizeof(float)), "hipMalloc(mlp)"); };
     al(&m->H1, rows * NH);
     al(&m->H2, rows * NH);
     al(&m->G3, rows * NO);
     al(&m->G2, rows * NH);
     al(&m->G1, rows * NH);
     al(&m->Xn, rows * NF);
-    hcheck(hipMalloc(&m->part, (size_t)((rows + RT - 1) / RT) * sizeof(double)), "hipMalloc(mlp)");
-    hcheck(hipMalloc(&m->gpart, (size_t)GCHUNKS * NP * sizeof(float)), "hipMalloc(mlp)");
-    hcheck(hipMalloc(&m->lacc, sizeof(double)), "hipMalloc(mlp)");
+    hcheck(dg::device_malloc(&m->part, (size_t)((rows + RT - 1) / RT) * sizeof(double)), "hipMalloc(mlp)");
+    hcheck(dg::device_malloc(&m->gpart, (size_t)GCHUNKS * NP * sizeof(float)), "hipMalloc(mlp)");
+    hcheck(dg::device_malloc(&m->lacc, sizeof(double)), "hipMalloc(mlp)");
     m->cap = rows;
 }
 
@@ -1060,15 +1060,15 @@ int dg_mlp_create(unsigned long long seed, dg_mlp** out) {
         m = new dg_mlp();
         hcheck(hipGetDevice(&m->device), "hipGetDevice");
         hcheck(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking), "hipStreamCreate");
-        hcheck(hipMalloc(&m->p, NP * sizeof(float)), "hipMalloc(mlp)");
-        hcheck(hipMalloc(&m->pb, NP * sizeof(uint16_t)), "hipMalloc(mlp)");
-        hcheck(hipMalloc(&m->img, IMG * sizeof(uint16_t)), "hipMalloc(mlp)");
-        hcheck(hipMalloc(&m->lane_img, LANE_IMG * sizeof(uint16_t)), "hipMalloc(mlp)");
+        hcheck(dg::device_malloc(&m->p, NP * sizeof(float)), "hipMalloc(mlp)");
+        hcheck(dg::device_malloc(&m->pb, NP * sizeof(uint16_t)), "hipMalloc(mlp)");
+        hcheck(dg::device_malloc(&m->img, IMG * sizeof(uint16_t)), "hipMalloc(mlp)");
+        hcheck(dg::device_malloc(&m->lane_img, LANE_IMG * sizeof(uint16_t)), "hipMalloc(mlp)");
         hcheck(dg::launch_zero(m->lane_img, LANE_IMG * sizeof(uint16_t), m->stream), "zero kernel");   // the padding
-        hcheck(hipMalloc(&m->g, NP * sizeof(float)), "hipMalloc(mlp)");
-        hcheck(hipMalloc(&m->m1, NP * sizeof(float)), "hipMalloc(mlp)");
-        hcheck(hipMalloc(&m->m2, NP * sizeof(float)), "hipMalloc(mlp)");
-        hcheck(hipMalloc(&m->xs, (2 * NF + NO) * sizeof(float)), "hipMalloc(mlp)");
+        hcheck(dg::device_malloc(&m->g, NP * sizeof(float)), "hipMalloc(mlp)");
+        hcheck(dg::device_malloc(&m->m1, NP * sizeof(float)), "hipMalloc(mlp)");
+        hcheck(dg::device_malloc(&m->m2, NP * sizeof(float)), "hipMalloc(mlp)");
+        hcheck(dg::device_malloc(&m->xs, (2 * NF + NO) * sizeof(float)), "hipMalloc(mlp)");
         // He-normal hidden layers, a small output layer (the correction
         // starts near zero), zero biases; identity scaling
         std::mt19937_64 rng(seed);
@@ -1296,8 +1296,8 @@ int dg_closure_step(dg_solver* s, dg_mlp* m, double dt_step, double bound, int n
         const long E = s->geo.E;
         // the corrections and the counter live on the solver handle from the
         // first call on (freed by dg_destroy)
-        if (!s->cl_C) hcheck(hipMalloc(&s->cl_C, (size_t)E * NO * sizeof(float)), "hipMalloc");
-        if (!s->cl_cnt) hcheck(hipMalloc(&s->cl_cnt, sizeof(unsigned long long)), "hipMalloc");
+        if (!s->cl_C) hcheck(dg::device_malloc(&s->cl_C, (size_t)E * NO * sizeof(float)), "hipMalloc");
+        if (!s->cl_cnt) hcheck(dg::device_malloc(&s->cl_cnt, sizeof(unsigned long long)), "hipMalloc");
         closure_steps(s, m, dt, bound, nsteps, s->cl_C, s->cl_cnt, n_fallback);
     });
 }

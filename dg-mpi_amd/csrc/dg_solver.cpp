@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstring>
 #include <exception>
+#include <memory>
 #include <new>
 #include <sstream>
 #include <string>
@@ -19,6 +20,72 @@
 
 #include "dg_solver_impl.hpp"
 
+
+namespace dg {
+
+namespace {
+
+// the scratch arrays held in the process (kept to the end: handles may be
+// destroyed after the static objects)
+struct Held {
+    std::mutex mu;
+    std::vector<Scratch*> all;
+};
+Held& held() {
+    static Held* h = new Held;
+    return *h;
+}
+
+// frees the device's scratch arrays; false if there was none
+bool take_back(int device) {
+    Held& h = held();
+    std::lock_guard<std::mutex> lk(h.mu);
+    bool any = false;
+    for (Scratch* q : h.all) {
+        std::lock_guard<std::mutex> ql(q->mu);
+        if (q->device != device || !q->p) continue;
+        // what is on the streams may still use it
+        if (hipDeviceSynchronize() != hipSuccess || hipFree(q->p) != hipSuccess) continue;
+        q->p = nullptr;
+        any = true;
+    }
+    return any;
+}
+
+}  // namespace
+
+hipError_t device_malloc(void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    int device = 0;
+    if (e != hipErrorOutOfMemory || hipGetDevice(&device) != hipSuccess || !take_back(device)) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
+void Scratch::take(size_t bytes, size_t arrays) {
+    size_t avail = 0, total = 0;
+    if (hipGetDevice(&device) != hipSuccess || hipMemGetInfo(&avail, &total) != hipSuccess ||
+        avail < bytes + arrays || hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+        return;
+    }
+    Held& h = held();
+    std::lock_guard<std::mutex> lk(h.mu);
+    h.all.push_back(this);
+}
+
+void Scratch::drop() {
+    {
+        Held& h = held();
+        std::lock_guard<std::mutex> lk(h.mu);
+        h.all.erase(std::remove(h.all.begin(), h.all.end(), this), h.all.end());
+    }
+    if (p) (void)hipFree(p);
+    p = nullptr;
+}
+
+}  // namespace dg
 
 namespace {
 
@@ -141,6 +208,9 @@ void step_once(dg_solver* s, double dt) {
     hip_check(launch_solver_stage(s, a, nullptr, s->stream), "stage kernel");
 }
 
+// the four registers and the carried rounding error
+size_t array_bytes(const dg_solver* s) { return s->ncoef * (4 * sizeof(double) + (s->cmp ? sizeof(float) : 0)); }
+
 // a new state starts without carried rounding error
 void clear_cmp(dg_solver* s) {
     if (s->cmp) hip_check(dg::launch_zero(s->cmp, s->ncoef * sizeof(float), s->stream), "zero kernel (cmp)");
@@ -193,8 +263,7 @@ void free_all(dg_solver* s) {
         if (p) (void)hipFree(p);
     if (s->cmp) (void)hipFree(s->cmp);
     s->cmp = nullptr;
-    if (s->faces) (void)hipFree(s->faces);
-    s->faces = nullptr;
+    s->faces.drop();
     if (s->frec) (void)hipFree(s->frec);
     s->frec = nullptr;
     s->nev = nullptr;
@@ -285,40 +354,34 @@ int create(const char* toml_text, const MeshInput* mesh, dg_solver** out) {
         hip_check(hipStreamCreateWithFlags(&s->own_stream, hipStreamNonBlocking), "hipStreamCreate");
         s->stream = s->own_stream;
         const size_t bytes = s->ncoef * sizeof(double);
-        hip_check(hipMalloc(&s->U0, bytes), "hipMalloc(U0)");
-        hip_check(hipMalloc(&s->Ua, bytes), "hipMalloc(Ua)");
-        hip_check(hipMalloc(&s->Ub, bytes), "hipMalloc(Ub)");
-        hip_check(hipMalloc(&s->acc, bytes), "hipMalloc(acc)");
-        hip_check(hipMalloc(&s->work, (size_t)s->geo.E * 6 * sizeof(double)), "hipMalloc(work)");
-        hip_check(hipMalloc(&s->dtab, sizeof(dg::KTables)), "hipMalloc(tables)");
+        hip_check(dg::device_malloc(&s->U0, bytes), "hipMalloc(U0)");
+        hip_check(dg::device_malloc(&s->Ua, bytes), "hipMalloc(Ua)");
+        hip_check(dg::device_malloc(&s->Ub, bytes), "hipMalloc(Ub)");
+        hip_check(dg::device_malloc(&s->acc, bytes), "hipMalloc(acc)");
+        hip_check(dg::device_malloc(&s->work, (size_t)s->geo.E * 6 * sizeof(double)), "hipMalloc(work)");
+        hip_check(dg::device_malloc(&s->dtab, sizeof(dg::KTables)), "hipMalloc(tables)");
         hip_check(hipMemcpy(s->dtab, &s->tab, sizeof(dg::KTables), hipMemcpyHostToDevice), "hipMemcpy(tables)");
         hip_check(dg::launch_zero(s->U0, bytes, s->stream), "zero kernel (U0)");
         if (cfg.compensated) {
-            hip_check(hipMalloc(&s->cmp, s->ncoef * sizeof(float)), "hipMalloc(cmp)");
+            hip_check(dg::device_malloc(&s->cmp, s->ncoef * sizeof(float)), "hipMalloc(cmp)");
             hip_check(dg::launch_zero(s->cmp, s->ncoef * sizeof(float), s->stream), "zero kernel (cmp)");
         }
-        if (const size_t fb = dg::two_pass_scratch_bytes(s->P, s->geo, s->geo.E)) {
-            // a case that fits the device without the scratch runs without it
-            if (hipMalloc(&s->faces, fb) != hipSuccess) {
-                (void)hipGetLastError();
-                s->faces = nullptr;
-            }
-        }
+        if (const size_t fb = dg::two_pass_scratch_bytes(s->P, s->geo, s->geo.E)) s->faces.take(fb, array_bytes(s));
         if (s->geo.mapped) {
             // upload the general-path tables, then form the per-element
             // inverse mass matrices (precompute_matrix_helpers,
             // src/solver/helpers.cpp:53-100)
-            hip_check(hipMalloc(&s->X, X.size() * sizeof(double)), "hipMalloc(X)");
+            hip_check(dg::device_malloc(&s->X, X.size() * sizeof(double)), "hipMalloc(X)");
             hip_check(hipMemcpy(s->X, X.data(), X.size() * sizeof(double), hipMemcpyHostToDevice), "hipMemcpy(X)");
-            hip_check(hipMalloc(&s->frec, ft.frec.size() * sizeof(unsigned)), "hipMalloc(frec)");
+            hip_check(dg::device_malloc(&s->frec, ft.frec.size() * sizeof(unsigned)), "hipMalloc(frec)");
             hip_check(hipMemcpy(s->frec, ft.frec.data(), ft.frec.size() * sizeof(unsigned), hipMemcpyHostToDevice),
                       "hipMemcpy(frec)");
             if (!ft.nev.empty()) {   // 3D only: 2D faces are straight
-                hip_check(hipMalloc(&s->nev, ft.nev.size() * sizeof(double)), "hipMalloc(nev)");
+                hip_check(dg::device_malloc(&s->nev, ft.nev.size() * sizeof(double)), "hipMalloc(nev)");
                 hip_check(hipMemcpy(s->nev, ft.nev.data(), ft.nev.size() * sizeof(double), hipMemcpyHostToDevice),
                           "hipMemcpy(nev)");
             }
-            hip_check(hipMalloc(&s->imm, (size_t)s->geo.E * nb * nb * sizeof(double)), "hipMalloc(imm)");
+            hip_check(dg::device_malloc(&s->imm, (size_t)s->geo.E * nb * nb * sizeof(double)), "hipMalloc(imm)");
             s->geo.X = s->X;
             s->geo.imm = s->imm;
             s->geo.frec = s->frec;
@@ -644,7 +707,7 @@ int dg_set_stream(dg_solver* s, void* stream) {
     return guarded(s, [&] {
         need(s, "solver");
         set_device(s);
-        std::lock_guard<std::mutex> lk(s->faces_mu);
+        std::lock_guard<std::mutex> lk(s->faces.mu);
         hip_check(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
         s->stream = stream ? (hipStream_t)stream : s->own_stream;
     });
@@ -671,9 +734,10 @@ struct dg_batch {
         std::vector<int> members;             // indices into cases
         dg::BatchCase* dcases = nullptr;      // device descriptors
         unsigned* blk_case = nullptr;         // device: case (within the group) of each block
-        // two-pass stage (faces != null; then blk_case holds the cases of the
-        // face pass's workgroups and, behind them, of the element pass's)
-        void* faces = nullptr;                // device: lifted fluxes of the group's faces
+        // two-pass stage (blk_case: behind the blocks, the cases of the face
+        // pass's workgroups and of the element pass's)
+        bool two_pass = false;
+        std::unique_ptr<dg::Scratch> faces;   // lifted fluxes of the group's cases
         unsigned pass_blocks[2] = {0, 0};     // workgroups of the face and of the element pass
         int variant = 0;                      // team-size variant of the launch (dg::batch_team)
         int cap = BRICK_CAPS[0];              // log2 edge cap of the element bricks of its cases
@@ -703,12 +767,21 @@ size_t group_face_bytes(const dg_batch::Group& g, const dg_solver* s) {
     return (dg::two_pass_scratch_bytes(g.P, s->geo, g.nblocks) + 255) & ~(size_t)255;
 }
 
+// keeps the batch's scratch from being taken back
+std::vector<std::unique_lock<std::mutex>> hold_scratch(const dg_batch* b) {
+    std::vector<std::unique_lock<std::mutex>> v;
+    for (const auto& g : b->groups) v.emplace_back(g.faces->mu);
+    return v;
+}
+
 // one RK4 stage of a group
 hipError_t launch_group_stage(const dg_batch* b, const dg_batch::Group& g, int variant, int stage, hipStream_t st) {
     const dg::KTables* t = b->cases[g.members[0]]->dtab;
-    if (g.faces)
-        return dg::launch_stage_two_pass_batch(g.P, g.flux, g.fp32, g.dcases, g.blk_case, g.pass_blocks[0],
-                                               g.blk_case + g.pass_blocks[0], g.pass_blocks[1], stage, t, st);
+    if (g.two_pass) {
+        const unsigned* face_case = g.blk_case + g.nblocks;
+        return dg::launch_stage_two_pass_batch(g.P, g.flux, g.fp32, g.dcases, face_case, g.pass_blocks[0],
+                                               face_case + g.pass_blocks[0], g.pass_blocks[1], stage, t, st);
+    }
     return dg::launch_stage_batch(g.P, g.flux, g.fp32, g.proj, variant, g.dcases, g.blk_case, g.nblocks, stage, t, st);
 }
 
@@ -737,8 +810,8 @@ void upload_group(dg_batch* b, dg_batch::Group& g) {
         for (int d = 0; d < 3; ++d) c.g.tile[d] = std::min(s->geo.tile[d], g.cap);
         c.first_block = first;
         first += s->geo.E;
-        if (g.faces) {
-            c.off_faces = off(g.faces) + (long long)face_bytes;
+        if (g.two_pass) {
+            c.off_faces = off(g.faces->p) + (long long)face_bytes;
             face_bytes += group_face_bytes(g, s);
             c.dv = make_box_div(s->geo);
             c.first_face = first_pass[0];
@@ -836,7 +909,7 @@ void tune(dg_batch* b) {
     for (auto& e : ev) (void)hipEventDestroy(e);
     for (auto& g : b->groups) {
         int best = 0;
-        if (g.faces) std::fill_n(g.ms_cand, NCAND, *std::min_element(g.ms_cand, g.ms_cand + NCAND));
+        if (g.two_pass) std::fill_n(g.ms_cand, NCAND, *std::min_element(g.ms_cand, g.ms_cand + NCAND));
         for (int c = 1; c < NCAND; ++c)
             if (g.ms_cand[c] < g.ms_cand[best]) best = c;
         g.variant = best & 1;
@@ -856,7 +929,7 @@ void free_batch(dg_batch* b) {
     for (auto& g : b->groups) {
         if (g.dcases) (void)hipFree(g.dcases);
         if (g.blk_case) (void)hipFree(g.blk_case);
-        if (g.faces) (void)hipFree(g.faces);
+        g.faces.reset();
         if (g.stream) (void)hipStreamDestroy(g.stream);
         if (g.done) (void)hipEventDestroy(g.done);
     }
@@ -923,25 +996,31 @@ int dg_batch_create(int num_cases, dg_solver* const* cases, dg_batch** out) {
             hip_check(hipEventCreateWithFlags(&b->groups[gi].done, hipEventDisableTiming), "hipEventCreate");
         }
         for (auto& g : b->groups) {
-            hip_check(hipMalloc(&g.dcases, g.members.size() * sizeof(dg::BatchCase)), "hipMalloc(batch cases)");
-            size_t face_bytes = 0;
-            for (int m : g.members) face_bytes += group_face_bytes(g, b->cases[m]);
-            if (face_bytes && hipMalloc(&g.faces, face_bytes) != hipSuccess) {
-                (void)hipGetLastError();      // no room for the scratch: the fused stage needs none
-                g.faces = nullptr;
+            hip_check(dg::device_malloc(&g.dcases, g.members.size() * sizeof(dg::BatchCase)), "hipMalloc(batch cases)");
+            size_t face_bytes = 0, bytes = 0;
+            for (int m : g.members) {
+                face_bytes += group_face_bytes(g, b->cases[m]);
+                bytes += array_bytes(b->cases[m]);
             }
-            // the case of each workgroup, of one launch or of both passes
+            // the case of each workgroup: of the fused launch, of the two passes
             std::vector<unsigned> bc;
-            for (int p = 0; p < (g.faces ? 2 : 1); ++p) {
+            for (int p = -1; p < (face_bytes ? 2 : 0); ++p) {
+                const size_t first = bc.size();
                 for (size_t m = 0; m < g.members.size(); ++m) {
                     const unsigned E = b->cases[g.members[m]]->geo.E;
-                    bc.insert(bc.end(), g.faces ? dg::two_pass_blocks(g.P, g.fp32, p, E) : E, (unsigned)m);
+                    bc.insert(bc.end(), p >= 0 ? dg::two_pass_blocks(g.P, g.fp32, p, E) : E, (unsigned)m);
                 }
-                if (g.faces) g.pass_blocks[p] = (unsigned)bc.size() - (p ? g.pass_blocks[0] : 0u);
+                if (p >= 0) g.pass_blocks[p] = (unsigned)(bc.size() - first);
             }
-            hip_check(hipMalloc(&g.blk_case, bc.size() * sizeof(unsigned)), "hipMalloc(batch blocks)");
+            hip_check(dg::device_malloc(&g.blk_case, bc.size() * sizeof(unsigned)), "hipMalloc(batch blocks)");
             hip_check(hipMemcpy(g.blk_case, bc.data(), bc.size() * sizeof(unsigned), hipMemcpyHostToDevice),
                       "hipMemcpy(batch blocks)");
+            g.faces.reset(new dg::Scratch);
+            if (face_bytes) g.faces->take(face_bytes, bytes);
+        }
+        const auto held = hold_scratch(b);
+        for (auto& g : b->groups) {
+            g.two_pass = g.faces->p != nullptr;
             upload_group(b, g);
         }
         b->dts.resize(b->cases.size());
@@ -964,7 +1043,8 @@ int dg_batch_step(dg_batch* b, int nsteps) {
         need(b, "batch");
         if (nsteps < 0) throw std::invalid_argument("nsteps < 0");
         hip_check(hipSetDevice(b->device), "hipSetDevice");
-        bool changed = false;
+        const auto held = hold_scratch(b);
+        bool changed = false, lost = false;
         for (size_t i = 0; i < b->cases.size(); ++i) {
             const dg_solver* s = b->cases[i];
             if (!(s->dt > 0.0))
@@ -978,6 +1058,12 @@ int dg_batch_step(dg_batch* b, int nsteps) {
             for (auto& g : b->groups) upload_group(b, g);
             for (size_t i = 0; i < b->cases.size(); ++i) b->dts[i] = b->cases[i]->dt;
         }
+        for (auto& g : b->groups)
+            if (g.two_pass && !g.faces->p) {       // taken back (device_malloc)
+                g.two_pass = false;
+                lost = true;
+            }
+        if (lost) capture_step(b);
         int n0 = 0;
         if (!b->tuned && nsteps >= TUNE_STEPS) {
             // the first steps of a long enough call pick each group's team

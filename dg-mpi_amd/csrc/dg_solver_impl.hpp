@@ -11,6 +11,34 @@
 #include "dg_config.hpp"
 #include "dg_kernels.hpp"
 
+namespace dg {
+
+// hipMalloc on the current device.  When the device is full, the two-pass
+// stage's scratch arrays on it are taken back first (their owners run the
+// fused stage from then on): no allocation of the library is refused for them.
+hipError_t device_malloc(void** p, size_t bytes);
+template <class T>
+hipError_t device_malloc(T** p, size_t bytes) {
+    return device_malloc(reinterpret_cast<void**>(p), bytes);
+}
+
+// Scratch of the two-pass stage, which its owner can do without.  mu is held
+// from the look at p until the launches that use it are on the stream (by a
+// batch until they are done): device_malloc of any thread may free it.
+struct Scratch {
+    void* p = nullptr;
+    int device = 0;
+    std::mutex mu;
+    // allocates it on the current device, where that leaves as much free as
+    // `arrays`, the bytes of the arrays it serves: the caller's own states of
+    // the case, or a second handle for it, then still fit
+    void take(size_t bytes, size_t arrays);
+    void drop();
+    ~Scratch() { drop(); }
+};
+
+}  // namespace dg
+
 struct dg_solver {
     dg::CaseConfig cfg;
     dg::KTables tab;
@@ -29,8 +57,7 @@ struct dg_solver {
     double* Ub = nullptr;
     double* acc = nullptr;             // RK accumulator
     float* cmp = nullptr;              // Stepper.compensated: rounding error of U0 (FP32)
-    void* faces = nullptr;             // scratch of the two-pass stage (null: the fused stage)
-    std::mutex faces_mu;               // its two launches go to the stream as one
+    dg::Scratch faces;                 // lifted fluxes of the two-pass stage (null: the fused stage)
     double* work = nullptr;            // per-element reduction output
     double* X = nullptr;               // mapped box: element node coordinates [E][8][3]
     double* imm = nullptr;             // mapped box: inverse mass matrices [E][nb][nb]
@@ -54,13 +81,14 @@ struct dg_solver {
 // needs no scratch.
 inline hipError_t launch_solver_stage(dg_solver* s, const dg::StageArgs& a, const float* corr, hipStream_t st) {
     const int flux = (int)s->cfg.flux;
-    if (s->faces) {
-        std::lock_guard<std::mutex> lk(s->faces_mu);
+    std::unique_lock<std::mutex> lk(s->faces.mu);
+    if (s->faces.p) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (a.mode != dg::MODE_RESIDUAL ||
             (st == s->stream && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone))
-            return dg::launch_stage_two_pass(s->P, flux, a, s->faces, corr, s->dtab, s->geo, st);
+            return dg::launch_stage_two_pass(s->P, flux, a, s->faces.p, corr, s->dtab, s->geo, st);
     }
+    lk.unlock();
     if (corr) return dg::launch_stage_corrected(s->P, flux, a, corr, s->dtab, s->geo, st);
     return dg::launch_stage(s->P, flux, a, s->dtab, s->geo, st);
 }

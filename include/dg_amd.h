@@ -83,7 +83,15 @@ typedef struct {
  * build the periodic mesh and the reference-element operators
  * (Solver<dim>::Solver + precompute_matrix_helpers,
  * src/solver/base.cpp:20-111) and allocate device state on the current
- * HIP device.  The state is left at zero; call dg_init_state. */
+ * HIP device.  The state is left at zero; call dg_init_state.
+ *   Memory: four registers of the state's size (4.5 with
+ * Stepper.compensated).  A 3D affine box of some thousand elements in FP64
+ * or the FP32 form also holds scratch for the two passes its stages run in,
+ * 3 / (p + 1) of the state (half of that in FP32), if that leaves as much
+ * again as the registers free.  When an allocation of the library fails, the
+ * scratch of all handles and batches on the device is freed and the
+ * allocation tried again; stages then run in one pass, slower and different
+ * in round-off. */
 int dg_create(const char* toml_text, dg_solver** out);
 
 /* The same for a hex mesh given as the arrays of the reference's mesh file
