@@ -55,11 +55,13 @@ bool take_back(int device) {
 }  // namespace
 
 hipError_t device_malloc(void** p, size_t bytes) {
-    const hipError_t e = hipMalloc(p, bytes);
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();                           // (a later launch would report it again)
     int device = 0;
-    if (e != hipErrorOutOfMemory || hipGetDevice(&device) != hipSuccess || !take_back(device)) return e;
-    (void)hipGetLastError();
-    return hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && take_back(device)) e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 void Scratch::take(size_t bytes, size_t arrays) {

@@ -126,3 +126,15 @@ def test_a_batch_goes_on_without_its_scratch():
                 assert np.max(np.abs(U1 - R)) <= step_tol(U0, R, order)
     for c in cases:
         c.close()
+
+
+def test_a_refused_handle_leaves_no_error_behind():
+    with Filler(ARRAYS // 2):
+        print("a handle that does not fit", flush=True)
+        with pytest.raises(dg_amd.DGError) as ei:
+            solver()
+        assert ei.value.status == 2 and "out of memory" in str(ei.value)
+        # the next call does not report it
+        with solver((4, 4, 4)) as s:
+            s.take_time_step()
+            assert np.all(np.isfinite(s.get_state()))
