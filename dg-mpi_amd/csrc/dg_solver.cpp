@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstring>
 #include <exception>
+#include <functional>
 #include <memory>
 #include <new>
 #include <sstream>
@@ -739,7 +740,10 @@ struct dg_batch {
         // two-pass stage (blk_case: behind the blocks, the cases of the face
         // pass's workgroups and of the element pass's)
         bool two_pass = false;
-        std::unique_ptr<dg::Scratch> faces;   // lifted fluxes of the group's cases
+        // lifted fluxes: a case's own scratch, or its share (from this byte
+        // on; -1: its own) of the group's array
+        std::vector<long long> share;
+        std::unique_ptr<dg::Scratch> faces;
         unsigned pass_blocks[2] = {0, 0};     // workgroups of the face and of the element pass
         int variant = 0;                      // team-size variant of the launch (dg::batch_team)
         int cap = BRICK_CAPS[0];              // log2 edge cap of the element bricks of its cases
@@ -769,11 +773,28 @@ size_t group_face_bytes(const dg_batch::Group& g, const dg_solver* s) {
     return (dg::two_pass_scratch_bytes(g.P, s->geo, g.nblocks) + 255) & ~(size_t)255;
 }
 
-// keeps the batch's scratch from being taken back
+// keeps the scratch of the batch and of its cases from being taken back
+// (locked in one order: batches of several threads may share cases)
 std::vector<std::unique_lock<std::mutex>> hold_scratch(const dg_batch* b) {
+    std::vector<dg::Scratch*> s;
+    for (const auto& g : b->groups) s.push_back(g.faces.get());
+    for (dg_solver* c : b->cases) s.push_back(&c->faces);
+    std::sort(s.begin(), s.end(), std::less<dg::Scratch*>());
     std::vector<std::unique_lock<std::mutex>> v;
-    for (const auto& g : b->groups) v.emplace_back(g.faces->mu);
+    for (dg::Scratch* q : s) v.emplace_back(q->mu);
     return v;
+}
+
+// scratch of the group's k-th case, or null
+char* case_faces(const dg_batch* b, const dg_batch::Group& g, size_t k) {
+    if (g.share[k] < 0) return static_cast<char*>(b->cases[g.members[k]]->faces.p);
+    return g.faces->p ? static_cast<char*>(g.faces->p) + g.share[k] : nullptr;
+}
+
+bool has_scratch(const dg_batch* b, const dg_batch::Group& g) {
+    for (size_t k = 0; k < g.share.size(); ++k)
+        if (!case_faces(b, g, k)) return false;
+    return !g.share.empty();
 }
 
 // one RK4 stage of a group
@@ -795,7 +816,6 @@ void upload_group(dg_batch* b, dg_batch::Group& g) {
     const char* base = reinterpret_cast<const char*>(g.dcases);
     auto off = [&](const void* p) { return (long long)(reinterpret_cast<const char*>(p) - base); };
     unsigned first = 0, first_pass[2] = {0, 0};
-    size_t face_bytes = 0;
     for (size_t k = 0; k < g.members.size(); ++k) {
         const dg_solver* s = b->cases[g.members[k]];
         BatchCase& c = h[k];
@@ -813,8 +833,7 @@ void upload_group(dg_batch* b, dg_batch::Group& g) {
         c.first_block = first;
         first += s->geo.E;
         if (g.two_pass) {
-            c.off_faces = off(g.faces->p) + (long long)face_bytes;
-            face_bytes += group_face_bytes(g, s);
+            c.off_faces = off(case_faces(b, g, k));
             c.dv = make_box_div(s->geo);
             c.first_face = first_pass[0];
             c.first_elem = first_pass[1];
@@ -999,14 +1018,20 @@ int dg_batch_create(int num_cases, dg_solver* const* cases, dg_batch** out) {
         }
         for (auto& g : b->groups) {
             hip_check(dg::device_malloc(&g.dcases, g.members.size() * sizeof(dg::BatchCase)), "hipMalloc(batch cases)");
+            // scratch for the cases without their own
             size_t face_bytes = 0, bytes = 0;
             for (int m : g.members) {
-                face_bytes += group_face_bytes(g, b->cases[m]);
-                bytes += array_bytes(b->cases[m]);
+                dg_solver* s = b->cases[m];
+                const size_t fb = group_face_bytes(g, s);
+                if (!fb) break;                    // (one answer for the group)
+                std::lock_guard<std::mutex> lk(s->faces.mu);
+                g.share.push_back(s->faces.p ? -1 : (long long)face_bytes);
+                if (!s->faces.p) face_bytes += fb;
+                bytes += array_bytes(s);
             }
             // the case of each workgroup: of the fused launch, of the two passes
             std::vector<unsigned> bc;
-            for (int p = -1; p < (face_bytes ? 2 : 0); ++p) {
+            for (int p = -1; p < (g.share.empty() ? 0 : 2); ++p) {
                 const size_t first = bc.size();
                 for (size_t m = 0; m < g.members.size(); ++m) {
                     const unsigned E = b->cases[g.members[m]]->geo.E;
@@ -1022,7 +1047,7 @@ int dg_batch_create(int num_cases, dg_solver* const* cases, dg_batch** out) {
         }
         const auto held = hold_scratch(b);
         for (auto& g : b->groups) {
-            g.two_pass = g.faces->p != nullptr;
+            g.two_pass = has_scratch(b, g);
             upload_group(b, g);
         }
         b->dts.resize(b->cases.size());
@@ -1061,7 +1086,7 @@ int dg_batch_step(dg_batch* b, int nsteps) {
             for (size_t i = 0; i < b->cases.size(); ++i) b->dts[i] = b->cases[i]->dt;
         }
         for (auto& g : b->groups)
-            if (g.two_pass && !g.faces->p) {       // taken back (device_malloc)
+            if (g.two_pass && !has_scratch(b, g)) {        // taken back (device_malloc)
                 g.two_pass = false;
                 lost = true;
             }

@@ -209,8 +209,8 @@ int dg_set_stream(dg_solver* s, void* stream);
  * differently in the batched kernel, and a group large enough takes its
  * stages in two passes though a case of it alone would not: both move
  * round-off only).  Cases: distinct handles on one device, 3D affine boxes
- * (no mesh, no warp), RK4.  The batch borrows the handles: destroy it
- * before them.  dg_batch_step waits for each case's stream before it starts
+ * (no mesh, no warp), RK4.  The batch borrows the handles, and the scratch
+ * of those that hold one (dg_create): destroy it before them.  dg_batch_step waits for each case's stream before it starts
  * and returns when the steps are done. */
 typedef struct dg_batch dg_batch;
 int dg_batch_create(int num_cases, dg_solver* const* cases, dg_batch** out);

@@ -138,3 +138,37 @@ def test_a_refused_handle_leaves_no_error_behind():
         with solver((4, 4, 4)) as s:
             s.take_time_step()
             assert np.all(np.isfinite(s.get_state()))
+
+
+def test_a_batch_uses_its_cases_scratch():
+    # both hold scratch of their own: 126 and 63 MB, twice the slack together
+    made = [(solver(ne), solver(ne)) for ne in ((64, 64, 64), (64, 32, 64), (3, 2, 1))]
+    batch_s, solo_s = [m[0] for m in made], [m[1] for m in made]
+    U0 = [s.get_state() for s in solo_s]
+    f0 = free_bytes()
+    with dg_amd.Batch(batch_s) as batch:
+        assert f0 - free_bytes() <= SLACK
+        for n in (1, 2, 7):                                 # replays of the captured step, then the tuned one
+            print(f"a batch on its cases' scratch, {n} steps", flush=True)
+            for sb, so, U in zip(batch_s, solo_s, U0):
+                sb.set_state(U)
+                so.set_state(U)
+            batch_s[0].take_time_step()                     # its scratch serves a step of its own in between
+            batch_s[0].set_state(U0[0])
+            batch.step(n)
+            for sb, so, U in zip(batch_s, solo_s, U0):
+                so.take_time_step(0.0, n)
+                R = so.get_state()
+                assert np.max(np.abs(sb.get_state() - R)) <= step_tol(U, R, 1, n)
+        # a case's scratch is taken back: the batch goes on without it
+        with Filler(ARRAYS + WORK - (48 << 20)):
+            with solver() as s:
+                s.take_time_step()
+        for sb, U in zip(batch_s, U0):
+            sb.set_state(U)
+        batch.step(7)
+        for sb, so, U in zip(batch_s, solo_s, U0):
+            R = so.get_state()
+            assert np.max(np.abs(sb.get_state() - R)) <= step_tol(U, R, 1, 7)
+    for s in batch_s + solo_s:
+        s.close()
