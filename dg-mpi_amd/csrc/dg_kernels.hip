@@ -3498,22 +3498,30 @@ hipError_t launch_stage(int P, int flux, const StageArgs& a, const KTables* t, c
 #if DG_PART == 3
 
 // Elements from which the two passes beat the fused stage, whose single
-// launch is the shorter one while launches and latency count (us, two passes /
-// fused, at the sizes on either side; a middle stage: FP64 p = 1 4096 12.1 /
-// 11.8, 8000 15.5 / 20.7; p = 2 1728 16.4 / 12.3, 4096 19.4 / 23.3; p = 3 1728
-// 24.7 / 20.3, 4096 34.6 / 38.4; FP32 p = 1 4096 12.4 / 10.2, 8000 15.0 / 15.7;
-// p = 2 4096 18.3 / 17.6, 8000 24.2 / 29.6; p = 4 19600 185 / 183, 32768 281 /
-// 384; p = 5 4096 81 / 79, 8000 145 / 151; the residual: FP64 p = 1 4624 11.8 /
-// 14.0, p = 2 2730 16.4 / 17.9, p = 5 2940 68.7 / 82.0; FP32 p = 3 4096 29.2 /
-// 27.3, 5832 33.1 / 36.7)
-unsigned two_pass_min_elements(int P, int fp32) {
-    static const unsigned lim[2][PMAX] = {{4608, 2560, 2816, 2816, 2816}, {7168, 5120, 5120, 24576, 6656}};
-    return P >= 1 && P <= PMAX ? lim[fp32 ? 1 : 0][P - 1] : ~0u;
+// launch is the shorter one while launches and latency count.  us, two passes /
+// fused, at the sizes on either side, the mean stage of an RK4 step: FP64 p = 1
+// 4096 12.1 / 11.2, 4913 12.4 / 15.0; p = 2 2197 15.5 / 14.8, 2744 16.2 / 17.7;
+// p = 3 2197 25.4 / 23.0, 2744 25.5 / 26.6; p = 4 1728 33.0 / 32.5, 2744 38.8 /
+// 45.5; p = 5 2744 69.4 / 71.4, 3375 75.9 / 89.0.  FP32, whose fused stage
+// takes half the LDS: p = 1 5832 12.7 / 12.7, 8000 14.1 / 15.0; p = 2 4096 17.7 /
+// 17.1, 5120 18.9 / 20.5; p = 3 5600 34.7 / 33.8, 6156 35.3 / 37.0; p = 4 13824
+// 125 / 124, 15625 141 / 146, 19683 173 / 191; p = 5 6859 124 / 122, 8000 136.0 /
+// 136.8, 12167 196 / 216.  The residual, whose element pass has no registers
+// to move, gains earlier: FP32 p = 3 5120 27.8 / 30.4, p = 5 6783 103 / 112.
+unsigned two_pass_min_elements(int P, int fp32, bool residual) {
+    static const unsigned lim[2][PMAX] = {{4608, 2560, 2816, 2816, 2816}, {7168, 5120, 5888, 14848, 8192}};
+    static const unsigned res[2][PMAX] = {{4608, 2560, 2816, 2816, 2816}, {7168, 5120, 5120, 14848, 6656}};
+    return P >= 1 && P <= PMAX ? (residual ? res : lim)[fp32 ? 1 : 0][P - 1] : ~0u;
 }
 
 size_t two_pass_scratch_bytes(int P, const KGeom& g, unsigned elements) {
-    if (g.dim != 3 || g.mapped || g.proj || P < 1 || P > PMAX || elements < two_pass_min_elements(P, g.fp32)) return 0;
+    if (g.dim != 3 || g.mapped || g.proj || P < 1 || P > PMAX || elements < two_pass_min_elements(P, g.fp32, true))
+        return 0;
     return (size_t)g.E * FACE_OUT(P) * (g.fp32 ? sizeof(float) : sizeof(double));
+}
+
+bool two_pass_steps(int P, const KGeom& g, unsigned elements) {
+    return elements >= two_pass_min_elements(P, g.fp32, false);
 }
 
 unsigned two_pass_blocks(int P, int fp32, int pass, unsigned E) {

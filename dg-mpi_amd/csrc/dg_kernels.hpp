@@ -169,9 +169,11 @@ hipError_t launch_stage(int P, int flux, const StageArgs& a, const KTables* t, c
 // FP64 and the FP32 form: every face's lifted flux once into `scratch`, then
 // the rest.  two_pass_scratch_bytes: the bytes of scratch for the case, 0
 // where launch_stage is the better one for a launch over `elements` elements
-// (the case's own, or all of a batch group) or the only one.  corr: the
-// correction of launch_stage_corrected, or null.
+// (the case's own, or all of a batch group) or the only one; two_pass_steps:
+// whether the two passes are the better ones for RK stages too and not for
+// the residual alone.  corr: the correction of launch_stage_corrected, or null.
 size_t two_pass_scratch_bytes(int P, const KGeom& g, unsigned elements);
+bool two_pass_steps(int P, const KGeom& g, unsigned elements);
 hipError_t launch_stage_two_pass(int P, int flux, const StageArgs& a, void* scratch, const float* corr,
                                  const KTables* t, const KGeom& g, hipStream_t st);
 // RK stage of an affine FP64 p = 1 box with dU = dt (M^-1 R + C): C the

@@ -770,6 +770,7 @@ thread_local std::string g_batch_error;
 
 // a case's bytes of its group's two-pass scratch array (0: fused stage)
 size_t group_face_bytes(const dg_batch::Group& g, const dg_solver* s) {
+    if (!dg::two_pass_steps(g.P, s->geo, g.nblocks)) return 0;
     return (dg::two_pass_scratch_bytes(g.P, s->geo, g.nblocks) + 255) & ~(size_t)255;
 }
 

@@ -84,8 +84,9 @@ inline hipError_t launch_solver_stage(dg_solver* s, const dg::StageArgs& a, cons
     std::unique_lock<std::mutex> lk(s->faces.mu);
     if (s->faces.p) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (a.mode != dg::MODE_RESIDUAL ||
-            (st == s->stream && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone))
+        if (a.mode != dg::MODE_RESIDUAL
+                ? dg::two_pass_steps(s->P, s->geo, s->geo.E)
+                : st == s->stream && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone)
             return dg::launch_stage_two_pass(s->P, flux, a, s->faces.p, corr, s->dtab, s->geo, st);
     }
     lk.unlock();
