@@ -2834,7 +2834,7 @@ void stage_batch_kernel(const BatchCase* __restrict__ cases,
     A.U0 = reinterpret_cast<const double*>(base + ou0);
     A.Uout = reinterpret_cast<double*>(const_cast<char*>(base) + oout);
     A.acc = reinterpret_cast<double*>(const_cast<char*>(base) + C->off_acc);
-    A.cmp = C->off_cmp >= 0 ? reinterpret_cast<float*>(const_cast<char*>(base) + C->off_cmp) : nullptr;
+    A.cmp = C->off_cmp != -1 ? reinterpret_cast<float*>(const_cast<char*>(base) + C->off_cmp) : nullptr;
     A.R = nullptr;
     A.dt = C->dt;
     A.alpha = stage == 2 ? 1.0 : 0.5;

@@ -149,7 +149,7 @@ constexpr int FACE_OUT(int P) { return 3 * NVAR * (P + 1) * (P + 1); }
 // first_block + E - 1).
 struct BatchCase {
     long long off_U0, off_Ua, off_Ub, off_acc;
-    long long off_cmp;       // compensation register, -1: plain update
+    long long off_cmp;       // compensation register (offsets may be negative), -1: plain update
     double dt;
     KGeom g;
     unsigned first_block;
