@@ -241,7 +241,9 @@ class Solver:
         return C.cast(p, C.c_void_p).value
 
     def get_residual(self, U_dev, R_dev, stream=None):
-        """R = volume - face at U (device pointers, [E][nb][5] FP64)."""
+        """R = volume - face at U (device pointers, [E][nb][5] FP64).  On the
+        handle's stream (set_stream; the default) large boxes take a faster
+        form, in FP64 different in round-off, than on any other or under capture."""
         self._check(lib().dg_residual(self._h, C.c_void_p(U_dev), C.c_void_p(R_dev),
                                       C.c_void_p(stream) if stream else None))
 

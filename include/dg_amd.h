@@ -156,7 +156,12 @@ int dg_state_device_ptr(dg_solver* s, double** dev);
 
 /* Residual R(U) = volume term - face term, not mass-inverted
  * (Solver::get_residual, src/solver/base.cpp:401-561).  U_dev and R_dev
- * are caller-owned device buffers of E*nb*5 doubles and must not alias. */
+ * are caller-owned device buffers of E*nb*5 doubles and must not alias.
+ *   On the handle's stream (dg_set_stream makes a caller's stream that) a
+ * handle with scratch (dg_create) takes two passes, about twice as fast; on
+ * any other stream, or under stream capture, the residual uses no memory of
+ * the handle's and runs in one.  In FP64 the two differ in round-off, in FP32
+ * they agree to the bit. */
 int dg_residual(dg_solver* s, const double* U_dev, double* R_dev, void* stream);
 
 /* dU = dt * M^-1 R per element (SolverTools::mult_inv_mass_matrix,
