@@ -768,9 +768,25 @@ namespace {
 
 thread_local std::string g_batch_error;
 
-// a case's bytes of its group's two-pass scratch array (0: fused stage)
+// Whether the group's stages are the faster ones in two passes: as for one box
+// of its elements, unless the cases leave the workgroups part empty (one holds
+// several elements, of one case), which costs more than the passes give: 352
+// boxes of 2^3 elements at p = 4, 7 and 1 elements in two workgroups, 223
+// against 200 us a step, 235 of 3 x 2 x 2, 7 and 5, 169 / 207; at p = 3, 5 and
+// 3, 119 / 115.
+bool group_two_pass(const dg_batch* b, const dg_batch::Group& g) {
+    const dg::KGeom& geo = b->cases[g.members[0]]->geo;
+    if (!dg::two_pass_steps(g.P, geo, g.nblocks) || !dg::two_pass_scratch_bytes(g.P, geo, g.nblocks)) return false;
+    for (int p = 0; p < 2; ++p) {
+        unsigned long long blocks = 0;
+        for (int m : g.members) blocks += dg::two_pass_blocks(g.P, g.fp32, p, b->cases[m]->geo.E);
+        if (3 * blocks > 4ull * dg::two_pass_blocks(g.P, g.fp32, p, g.nblocks)) return false;
+    }
+    return true;
+}
+
+// a case's bytes of its group's two-pass scratch array
 size_t group_face_bytes(const dg_batch::Group& g, const dg_solver* s) {
-    if (!dg::two_pass_steps(g.P, s->geo, g.nblocks)) return 0;
     return (dg::two_pass_scratch_bytes(g.P, s->geo, g.nblocks) + 255) & ~(size_t)255;
 }
 
@@ -1021,15 +1037,14 @@ int dg_batch_create(int num_cases, dg_solver* const* cases, dg_batch** out) {
             hip_check(dg::device_malloc(&g.dcases, g.members.size() * sizeof(dg::BatchCase)), "hipMalloc(batch cases)");
             // scratch for the cases without their own
             size_t face_bytes = 0, bytes = 0;
-            for (int m : g.members) {
-                dg_solver* s = b->cases[m];
-                const size_t fb = group_face_bytes(g, s);
-                if (!fb) break;                    // (one answer for the group)
-                std::lock_guard<std::mutex> lk(s->faces.mu);
-                g.share.push_back(s->faces.p ? -1 : (long long)face_bytes);
-                if (!s->faces.p) face_bytes += fb;
-                bytes += array_bytes(s);
-            }
+            if (group_two_pass(b, g))
+                for (int m : g.members) {
+                    dg_solver* s = b->cases[m];
+                    std::lock_guard<std::mutex> lk(s->faces.mu);
+                    g.share.push_back(s->faces.p ? -1 : (long long)face_bytes);
+                    if (!s->faces.p) face_bytes += group_face_bytes(g, s);
+                    bytes += array_bytes(s);
+                }
             // the case of each workgroup: of the fused launch, of the two passes
             std::vector<unsigned> bc;
             for (int p = -1; p < (g.share.empty() ? 0 : 2); ++p) {
